@@ -1,15 +1,16 @@
 """Performance cases of the flash-attention forward: what a program that uses this library has it
 compute, through the public Python entry points (flash_launch, and HIP graphs of such launches).
 
-A case is one call, or the launches of a stack of layers captured once into a HIP graph and replayed
-(the way short launches are issued when latency matters):
+A case is one call, or the calls of a stack of layers: made one by one, or captured once into a HIP
+graph and replayed (the way short launches are issued when latency matters):
   batch_heads, seq_len, head_dim, causal, dtype ("f16" | "bf16")
   layout   "dense"  packed slices
            "rows"   every row padded by 8 elements (16-byte aligned rows)
            "odd"    slices padded by 17/19/23/29 elements (Q/K/V/O), as the reference's smoke cases pad
                     theirs: slice bases have no common alignment beyond the element's own
   sigma    standard deviation of Q and K (1: ordinary logits; 3: sharp ones, where few keys dominate)
-  layers   0: one direct call; n > 0: a captured graph of n calls, each on tensors of its own
+  layers   calls of one pass, each on tensors of its own
+  graph    the calls are a captured graph, replayed once a pass
 """
 
 import math
@@ -30,21 +31,23 @@ ODD_PADS = (17, 19, 23, 29)
 DTYPES = {"f16": torch.float16, "bf16": torch.bfloat16}
 
 
-def _case(name, batch_heads, seq_len, head_dim, causal, dtype="f16", layout="dense", sigma=1.0, layers=0):
+def _case(name, batch_heads, seq_len, head_dim, causal, dtype="f16", layout="dense", sigma=1.0, layers=1,
+          graph=False):
     return {"name": name, "batch_heads": batch_heads, "seq_len": seq_len, "head_dim": head_dim, "causal": causal,
-            "dtype": dtype, "layout": layout, "sigma": sigma, "layers": layers}
+            "dtype": dtype, "layout": layout, "sigma": sigma, "layers": layers, "graph": graph}
 
 
 def listed():
     return [
-        # One call on the smallest problem (a 32-token prompt, one head): the cost of a call itself.
-        _case("single_tiny", 1, 32, 16, False),
+        # The smallest calls (a 32-token prompt, one head), made one by one through a stack of layers:
+        # the cost of a call itself.
+        _case("calls_tiny", 1, 32, 16, False, layers=LAYERS),
         # A short prompt through a captured stack of layers, rows padded to a pitch of 40.
-        _case("stack_short_rows", 8, 128, 32, True, layout="rows", layers=LAYERS),
+        _case("stack_short_rows", 8, 128, 32, True, layout="rows", layers=LAYERS, graph=True),
         # The same kind of stack on slices with the reference's odd pads, ragged length.
-        _case("stack_short_odd", 8, 250, 32, True, layout="odd", layers=LAYERS),
+        _case("stack_short_odd", 8, 250, 32, True, layout="odd", layers=LAYERS, graph=True),
         # The headline shape: a 1024-token causal prefill of 8 heads, as a captured stack.
-        _case("stack_headline", 8, 1024, 64, True, layers=LAYERS),
+        _case("stack_headline", 8, 1024, 64, True, layers=LAYERS, graph=True),
         # Many short ragged sequences in a batch (192 heads x 333 tokens), bf16.
         _case("batch_ragged_bf16", 192, 333, 64, True, dtype="bf16"),
         # An encoder-style full attention at a mid size on odd slices.
@@ -80,8 +83,9 @@ def draw(rng):
         most //= 4
     pairs = seq_len * seq_len // (2 if causal else 1)
     batch_heads = max(1, min(batch_heads, most // pairs))
-    layers = LAYERS if batch_heads * pairs <= 8 * 1024 * 1024 and rng.random() < 0.8 else 0
-    case = _case("", batch_heads, seq_len, head_dim, causal, dtype, layout, rng.choice((1.0, 1.0, 3.0)), layers)
+    short = batch_heads * pairs <= 8 * 1024 * 1024
+    case = _case("", batch_heads, seq_len, head_dim, causal, dtype, layout, rng.choice((1.0, 1.0, 3.0)),
+                 LAYERS if short else 1, short and rng.random() < 0.75)
     del case["name"]
     return case
 
@@ -132,7 +136,7 @@ def _inputs(case, seed):
     """Q, K, V as [calls, batch_heads * slice stride] tensors, paddings filled like the rest."""
     gen = torch.Generator(device="cuda")
     gen.manual_seed(seed)
-    calls = max(1, case["layers"])
+    calls = case["layers"]
     _, strides = _strides(case)
     out = []
     for which, stride in zip("qkv", strides):
@@ -145,7 +149,7 @@ def prepare(case, seed):
     module, stream = _context()
     q, k, v = _inputs(case, seed)
     row, strides = _strides(case)
-    calls = max(1, case["layers"])
+    calls = case["layers"]
     o = torch.zeros(calls, case["batch_heads"] * strides[3], device="cuda", dtype=torch.float32)
     opts = nc.options(batch_heads=case["batch_heads"], seq_len=case["seq_len"], head_dim=case["head_dim"],
                       q_stride=strides[0], k_stride=strides[1], v_stride=strides[2], o_stride=strides[3],
@@ -153,7 +157,7 @@ def prepare(case, seed):
                       dtype=case["dtype"])
     state = {"module": module, "opts": opts, "tensors": (q, k, v, o), "o": o,
              "buffers": [tuple(_Buffer(t[i]) for t in (q, k, v, o)) for i in range(calls)], "stack": None}
-    if case["layers"]:
+    if case["graph"]:
         torch.cuda.synchronize()  # the graph's stream does not wait for the fills above
 
         def body():
@@ -168,12 +172,13 @@ def run(state):
     if state["stack"] is not None:
         state["stack"]()
     else:
-        nc.flash_launch(state["module"], *state["buffers"][0], state["opts"])
+        for bufs in state["buffers"]:
+            nc.flash_launch(state["module"], *bufs, state["opts"])
     return state["o"]
 
 
 def work(case):
-    calls, s, d = max(1, case["layers"]), case["seq_len"], case["head_dim"]
+    calls, s, d = case["layers"], case["seq_len"], case["head_dim"]
     pairs = s * (s + 1) // 2 if case["causal"] else s * s
     return {"bytes": calls * case["batch_heads"] * s * d * (3 * 2 + 4),
             "flops": calls * case["batch_heads"] * pairs * d * 4}
@@ -191,7 +196,7 @@ def tolerance(case):
 def exact(case, seed):
     """The attention of the same inputs in float64, paddings of O as prepare() leaves them."""
     row, strides = _strides(case)
-    bh, s, d, calls = case["batch_heads"], case["seq_len"], case["head_dim"], max(1, case["layers"])
+    bh, s, d, calls = case["batch_heads"], case["seq_len"], case["head_dim"], case["layers"]
     q, k, v = (t.as_strided((calls, bh, s, d), (bh * st, st, row, 1))
                for t, st in zip(_inputs(case, seed), strides))
     out = torch.zeros(calls, bh * strides[3], device="cuda", dtype=torch.float64)
