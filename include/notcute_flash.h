@@ -248,7 +248,7 @@ typedef struct nc_flash_kernel_selection {
     uint32_t block_n;           /* keys staged per workgroup iteration */
     uint32_t kv_splits;         /* waves that share one query tile and split its keys */
     uint32_t lds_bytes;         /* static LDS of the kernel */
-    uint32_t aligned;           /* 1: 16-byte vector path, 0: element-wise path for odd strides */
+    uint32_t aligned;           /* 1: every Q/K/V row is 16-byte and every O row float4 aligned */
     uint64_t scratch_bytes;     /* device scratch the kernel needs (pair-split kernels), else 0 */
 } nc_flash_kernel_selection;
 

@@ -78,6 +78,11 @@ struct Variant {
 // Two 32-key sub-tiles per wave per block ("t2": 32*NS*2 keys per block).
 #define PIPE2(D, NQ, NS, P, C, T, BF) {"nc_flash_fwd_d" #D "_q" #NQ "s" #NS "p" #P "t2_" C T, D, NQ, NS, P, 2, \
                                        C[0] == 'c', true, Family::kPipe, BF}
+// Slices at any 2-byte alignment (SUF: "" or "t2").
+#define PIPEU(D, NQ, NS, P, SUB, SUF, C, T, BF) {"nc_flash_fwd_d" #D "_q" #NQ "s" #NS "p" #P SUF "_" C "_unaligned" T, \
+                                                 D, NQ, NS, P, SUB, C[0] == 'c', false, Family::kPipe, BF}
+#define PIPEU2(D, NQ, NS, P, SUB, SUF, T, BF) PIPEU(D, NQ, NS, P, SUB, SUF, "full", T, BF), \
+    PIPEU(D, NQ, NS, P, SUB, SUF, "causal", T, BF)
 #define GEN(D, C, A, SUF, T, BF) {"nc_flash_fwd_d" #D "_m64_" C SUF T, D, 2, 2, 1, 1, C[0] == 'c', A, \
                                   Family::kGeneric, BF}
 // The generic body in other geometries (32 rows x 8 key splits; 128 rows x 2 key splits).
@@ -102,7 +107,12 @@ struct Variant {
     GENG2(16, 1, 8, T, BF), GENG2(32, 1, 8, T, BF), GENG2(64, 1, 8, T, BF), GENG2(64, 4, 2, T, BF),          \
     PIPE(64, 1, 8, 1, "full", T, BF), PIPE(64, 1, 8, 1, "causal", T, BF), PIPE(32, 1, 8, 1, "full", T, BF),   \
     PIPE(32, 1, 8, 1, "causal", T, BF), PIPE(16, 1, 8, 1, "full", T, BF), PIPE(16, 1, 8, 1, "causal", T, BF), \
-    PIPED4(64, T, BF), PIPED4(32, T, BF), PIPED4(16, T, BF)
+    PIPED4(64, T, BF), PIPED4(32, T, BF), PIPED4(16, T, BF),                                                  \
+    PIPEU2(64, 8, 1, 2, 2, "t2", T, BF), PIPEU2(64, 4, 1, 2, 2, "t2", T, BF), PIPEU2(64, 2, 4, 2, 1, "", T, BF), \
+    PIPEU2(64, 1, 8, 2, 1, "", T, BF), PIPEU2(64, 1, 8, 1, 1, "", T, BF), PIPEU2(32, 4, 1, 2, 1, "", T, BF),   \
+    PIPEU2(32, 2, 4, 2, 1, "", T, BF), PIPEU2(32, 1, 8, 2, 1, "", T, BF), PIPEU2(32, 1, 8, 1, 1, "", T, BF),   \
+    PIPEU2(16, 4, 1, 2, 2, "t2", T, BF), PIPEU2(16, 2, 4, 2, 1, "", T, BF), PIPEU2(16, 1, 8, 2, 1, "", T, BF), \
+    PIPEU2(16, 1, 8, 1, 1, "", T, BF)
 
 const Variant kVariants[] = {VARIANTS("", false), VARIANTS("_bf16", true)};
 #undef VARIANTS
@@ -111,6 +121,8 @@ const Variant kVariants[] = {VARIANTS("", false), VARIANTS("_bf16", true)};
 #undef PIPEX
 #undef PIPED
 #undef PIPED4
+#undef PIPEU
+#undef PIPEU2
 #undef GEN
 #undef GENG
 #undef GENG2
@@ -118,7 +130,7 @@ const Variant kVariants[] = {VARIANTS("", false), VARIANTS("_bf16", true)};
 const Variant *find_pipe(uint32_t d, uint32_t nq, uint32_t ns, bool causal, bool bf16) {
     for (const auto &v : kVariants)
         if (v.family == Family::kPipe && v.d == d && v.nq == nq && v.ns == ns && v.causal == causal && v.bf16 == bf16 &&
-            !v.xsplit && !v.dense)
+            !v.xsplit && !v.dense && v.aligned)
             return &v;
     return nullptr;
 }
@@ -127,7 +139,16 @@ const Variant *find_pipe(uint32_t d, uint32_t nq, uint32_t ns, bool causal, bool
 const Variant *find_pipe_stages(uint32_t d, uint32_t nq, uint32_t ns, uint32_t nstage, bool causal, bool bf16) {
     for (const auto &v : kVariants)
         if (v.family == Family::kPipe && v.d == d && v.nq == nq && v.ns == ns && v.nstage == nstage &&
-            v.causal == causal && v.bf16 == bf16 && !v.xsplit && !v.dense)
+            v.causal == causal && v.bf16 == bf16 && !v.xsplit && !v.dense && v.aligned)
+            return &v;
+    return nullptr;
+}
+
+// The kernel of a pipelined one's geometry and ring depth for rows at any 2-byte alignment.
+const Variant *find_unaligned(const Variant &base, uint32_t nstage) {
+    for (const auto &v : kVariants)
+        if (v.family == Family::kPipe && !v.aligned && v.d == base.d && v.nq == base.nq && v.ns == base.ns &&
+            v.nstage == nstage && v.causal == base.causal && v.bf16 == base.bf16)
             return &v;
     return nullptr;
 }
@@ -172,7 +193,7 @@ const Variant *find_generic(uint32_t d, uint32_t nq, uint32_t ns, bool causal, b
     return nullptr;
 }
 
-// Geometry of the generic kernels (rows past 16-byte alignment or past 32-bit offsets), from GPU
+// Geometry of the generic kernels (rows past 32-bit offsets, odd or unequal K/V row strides), from GPU
 // timings of the three on 132 shapes (d 16/32/64, BH 1-128, S 256-8192, causal and not), where
 // these picks come within 0.6 % of the per-shape best on average and the 64-row kernel alone
 // averaged 1.30-1.83x: 32 rows x 8 key splits while the grid is small, 128 x 2 for large d=64
@@ -391,7 +412,17 @@ const Variant *choose_pipe_layout(const nc_flash_options &o) {
     return best;
 }
 
-bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+// Slices at odd elements: the pipelined choice in its `_unaligned` form (two stages where that has
+// three). Measured on MI355X with the reference's odd slice pads (17, 19, 23, 29), generic kernels ->
+// these: BH=8 S=1024 d=64 causal 19.3 -> 7.5 us, BH=16 S=1500 d=64 43.6 -> 20.3, BH=32 S=4096 d=64
+// 267 -> 152, BH=128 S=1000 d=32 causal 30.8 -> 21.4, BH=64 S=2048 d=16 88 -> 51, BH=3 S=49 d=16 causal
+// 3.21 -> 3.20 us; 16-byte aligned slices of the same shapes run 5.6, 18.0, 154, 19.6, 51 and 2.5 us.
+const Variant *choose_unaligned(const nc_flash_options &o) {
+    const Variant *v = choose_pipe(o);
+    return v ? find_unaligned(*v, v->nq == 1 ? v->nstage : 2) : nullptr;
+}
+
+uintptr_t address(const void *p) { return reinterpret_cast<uintptr_t>(p); }
 
 // Every tensor a stack of packed slices: slice stride seq_len * d elements, row stride d.
 bool dense_layout(const nc_flash_options &o) {
@@ -401,7 +432,8 @@ bool dense_layout(const nc_flash_options &o) {
            o.k_stride == slice && o.v_stride == slice && o.o_stride == slice;
 }
 
-int select_impl(const nc_flash_options *opts, bool vec_ok, nc_flash_kernel_selection *out) {
+// low: the low address bits that any of Q, K, V sets, olow: O's.
+int select_impl(const nc_flash_options *opts, uintptr_t low, uintptr_t olow, nc_flash_kernel_selection *out) {
     if (!out) return NC_ERROR_INVALID_VALUE;
     int st = nc_flash_validate(opts);
     if (st) return st;
@@ -413,15 +445,24 @@ int select_impl(const nc_flash_options *opts, bool vec_ok, nc_flash_kernel_selec
     const bool strides_ok = o.q_stride % 8 == 0 && o.k_stride % 8 == 0 && o.v_stride % 8 == 0 &&
                             o.o_stride % 4 == 0 && rows[0] % 8 == 0 && rows[1] % 8 == 0 && rows[2] % 8 == 0 &&
                             rows[3] % 4 == 0;
-    const bool aligned = vec_ok && strides_ok;
+    const bool aligned = ((low | olow) & 15u) == 0 && strides_ok;
+    // The pipelined kernels' 16-byte loads need every Q/K/V row to start at a dword (measured: the rate
+    // of aligned ones, buffer->LDS 147 GB/s per CU either way), their stores an O row at a float; their `_unaligned` forms take Q, K and V at any element, with one even row stride for K and V.
+    const bool o_floats = (olow & 3u) == 0;
+    const bool dwords = o_floats && (low & 3u) == 0 &&
+                        ((o.q_stride | o.k_stride | o.v_stride | rows[0] | rows[1] | rows[2]) & 1u) == 0;
+    const bool elements = o_floats && (low & 1u) == 0 && (rows[1] & 1u) == 0 && rows[1] == rows[2];
     // The pipelined kernels address each Q/K/V slice with 32-bit buffer offsets, including up to
     // one block (<= 256 rows) past seq_len.
     uint64_t max_row = rows[0] > rows[1] ? rows[0] : rows[1];
     max_row = max_row > rows[2] ? max_row : rows[2];
     const bool offsets_fit = max_row < (1ull << 30) && (o.seq_len + 512) * max_row * 2 < (1ull << 31);
-    const Variant *v = (aligned && offsets_fit)
-                           ? choose_pipe(o)
-                           : choose_generic(o, aligned);
+    const Variant *v = offsets_fit && dwords     ? choose_pipe(o)
+                       : offsets_fit && elements ? choose_unaligned(o)
+                                                 : choose_generic(o, aligned);
+    // A grid past the dispatch packet's work-items (below) on more threads than the generic kernel's.
+    if (v && !aligned && (o.seq_len + v->bm() - 1) / v->bm() > 0xffffffffull / v->threads() / o.batch_heads)
+        v = choose_generic(o, aligned);
     if (!v) return NC_ERROR_NOT_FOUND;
     // Long causal sequences over few heads on the private-staging kernel: pair the light and heavy
     // query blocks so that every workgroup takes about half the heaviest block's keys. It pays once
@@ -430,7 +471,9 @@ int select_impl(const nc_flash_options *opts, bool vec_ok, nc_flash_kernel_selec
     // BH=1 S=8192 23.4 -> 18.6 us, BH=2 S=4096 13.4 -> 12.3 us, but c3 (32 query blocks) 5.9 -> 7.5 us
     // and grids beyond 256 workgroups slower too.
     const uint64_t nqb32 = (o.seq_len + 31) / 32;
-    if (v->family == Family::kPipe && v->causal && v->nq == 1 && v->d == 64 && nqb32 >= 96 &&
+    // Only on 16-byte aligned slices: its scratch must not be shared by launches that overlap, and the
+    // other layouts' kernels have never needed any.
+    if (v->family == Family::kPipe && aligned && v->causal && v->nq == 1 && v->d == 64 && nqb32 >= 96 &&
         nqb32 * o.batch_heads <= 256 && xsplit_pairs(o.batch_heads, o.seq_len) <= NC_XS_MAX_PAIRS) {
         const Variant *x = find_xsplit(v->d, v->bf16);
         if (x) v = x;
@@ -444,7 +487,7 @@ int select_impl(const nc_flash_options *opts, bool vec_ok, nc_flash_kernel_selec
     // kernel with the argument block (interleaved graph replays, bitwise-identical output): c3 5.71
     // -> 5.49 us, BH=8 S=1536 causal 8.50 -> 8.16 us, BH=8 S=2048 causal 10.80 -> 10.52 us. Grid
     // (8, BH/8, nqb) or (BH, 1, nqb): the same workgroups in the same linear order as the 1-D grid.
-    if (v->family == Family::kPipe && v->nq == 1 && !v->xsplit && dense_layout(o) && nqb <= 65535) {
+    if (v->family == Family::kPipe && aligned && v->nq == 1 && !v->xsplit && dense_layout(o) && nqb <= 65535) {
         const Variant *dv = find_dense(*v);
         const uint64_t bh = o.batch_heads;
         if (dv && (bh % 8 == 0 ? bh / 8 <= 65535 : bh <= 0x7fffffffu)) {  // grid y, z <= 65535; x < 2^31
@@ -516,12 +559,12 @@ int nc_flash_validate(const nc_flash_options *opts) {
 }
 
 int nc_flash_select_kernel(const nc_flash_options *opts, nc_flash_kernel_selection *out) {
-    return select_impl(opts, true, out);
+    return select_impl(opts, 0, 0, out);
 }
 
 int nc_flash_select_kernel_for(const nc_flash_options *opts, const void *q, const void *k, const void *v,
                                const void *o, nc_flash_kernel_selection *out) {
-    return select_impl(opts, aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o), out);
+    return select_impl(opts, address(q) | address(k) | address(v), address(o), out);
 }
 
 int nc_flash_pack_args(const nc_flash_options *opts, const nc_flash_kernel_selection *sel, const uint16_t *q,

@@ -27,8 +27,8 @@
 //     the workgroup's last query are never staged. Heavy (late) query blocks are dispatched first and
 //     workgroups of the same heads are kept on one XCD so their K/V stay in that XCD's L2.
 //   * exp is v_exp_f32 on log2-scaled scores (scale * log2(e) folded into one multiply).
-// The generic family (flash_fwd_body: any 16-byte aligned layout, 64-bit addressing, and element-wise
-// variants for unaligned ones) stages K/V through registers and stores V^T transposed in LDS with
+// The generic family (flash_fwd_body: 64-bit addressing, and element-wise variants for odd or unequal
+// K/V row strides and unaligned slices of that size) stages K/V through registers and stores V^T transposed in LDS with
 // keys permuted so each A-operand fetch is one ds_read_b128. The pipelined family
 // (flash_fwd_pipe_body, the fast path) streams K/V with buffer->LDS DMA into a ring and reads V^T
 // with ds_read_b64_tr_b16; it is described where it is defined.
@@ -444,7 +444,7 @@ __device__ __forceinline__ void flash_fwd_body(const nc_flash_kernel_args &a) {
 
 
 // ---------------------------------------------------------------------------------------------
-// Pipelined variant (16-byte aligned rows, slices below 2 GiB): K and V stream through an
+// Pipelined variant (dword-aligned rows, in its UN form any slices; below 2 GiB): K and V stream through an
 // NSTAGE-deep LDS ring by direct buffer->LDS loads (buffer_load_dwordx4 ... lds), so no VGPRs or
 // ds_write instructions are spent on staging and NSTAGE-1 blocks are always in flight. The buffer
 // descriptors cover exactly each slice's active rows, so key rows past seq_len read as zero
@@ -697,7 +697,22 @@ constexpr int pipe_lds_bytes() {
 #endif
 
 // slot_of(batch_heads) gives the workgroup's PipeSlot (called once the arguments are checked).
-template <int D, int NQ, int NS, bool CAUSAL, int NSTAGE, int SUB, bool BF, bool XS = false, typename SlotFn>
+//
+// UN (the `_unaligned` kernels): slices at any 2-byte alignment, K and V rows the same even number of
+// elements apart. A 16-byte load at an odd element runs at 37 GB/s per CU, at a dword-aligned address
+// at 138 GB/s, buffer->LDS at 147 (measured, L2-resident data), so the ring loads take every chunk
+// from its address rounded down to a dword. A slice that starts in the upper half of a dword then
+// arrives one element early: position e of a staged row holds column e - 1, position 0 an element of
+// the row before, and column D - 1 is missing. It goes to position 0 (one 2-byte load and one
+// ds_write_b16 per row), so the row is rotated by one, which costs nothing more: S^T is the same
+// with Q rotated alike when it is loaded, and the rotated O^T rows are put right at the store. An
+// even slice in the same launch skips all of it (kodd, vodd are uniform).
+// Odd slice pads, us: element-wise generic kernels / staging through registers with a funnel shift
+// per chunk (148-176 VGPRs, half the workgroups per CU) / shifting each chunk in place in LDS / this:
+// BH=8 S=1024 d=64 causal 19.3 / 8.7 / 11.1 / 7.5, BH=32 S=4096 d=64 267 / 209 / 181 / 152, BH=16 S=1500
+// d=64 35.4 / 31.0 / 27.9 / 20.3 (16-byte aligned slices: 5.6, 154, 18.0).
+template <int D, int NQ, int NS, bool CAUSAL, int NSTAGE, int SUB, bool BF, bool XS = false, bool UN = false,
+          typename SlotFn>
 __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &a, char *smem, SlotFn &&slot_of) {
     using C = PipeCfg<D, NQ, NS, NSTAGE, SUB>;
     using SW = Swz<D>;
@@ -787,12 +802,32 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     const int qw_last = min(qw0 + 31, S - 1);
 
     const uint32_t qrb = (uint32_t)a.q_row_stride * 2, krb = (uint32_t)a.k_row_stride * 2;
-    const uint32_t vrb = (uint32_t)a.v_row_stride * 2;
+    const uint32_t vrb = UN ? krb : (uint32_t)a.v_row_stride * 2;  // UN: one row stride, so K and V share offsets
     const uint32_t qspan = (uint32_t)((S - 1) * (uint64_t)a.q_row_stride + D) * 2;
     const uint32_t kspan = (uint32_t)((S - 1) * (uint64_t)a.k_row_stride + D) * 2;
     const uint32_t vspan = (uint32_t)((S - 1) * (uint64_t)a.v_row_stride + D) * 2;
-    const __amdgpu_buffer_rsrc_t kr = make_rsrc(a.k + (size_t)head * a.k_stride, kspan);
-    const __amdgpu_buffer_rsrc_t vr = make_rsrc(a.v + (size_t)head * a.v_stride, vspan);
+    // UN: a slice's descriptor starts at the dword that holds its first element and ends before the one
+    // that holds nothing but its last (column D - 1 of the last row, which the ring loads do not take,
+    // beside an element past the slice, which must not reach the padding row after it: a weight of
+    // zero does not cancel an infinity).
+    auto slice_rsrc = [](const uint16_t *p, uint32_t span) {
+        if constexpr (UN) {
+            const uint32_t phase = (uint32_t)((uintptr_t)p & 2);
+            return make_rsrc((const void *)((uintptr_t)p - phase), (span + phase) & ~3u);
+        } else {
+            return make_rsrc(p, span);
+        }
+    };
+    // The same with the last element's dword (two bytes past the slice at most, in the same dword).
+    auto edge_rsrc = [](const uint16_t *p, uint32_t span) {
+        return make_rsrc((const void *)((uintptr_t)p - ((uintptr_t)p & 2)), span + 4u);
+    };
+    const uint16_t *kh = a.k + (size_t)head * a.k_stride, *vh = a.v + (size_t)head * a.v_stride;
+    const bool kodd = UN && ((uintptr_t)kh & 2) != 0, vodd = UN && ((uintptr_t)vh & 2) != 0;
+    // other row strides: the host launches the generic kernels
+    if (UN && ((krb & 2u) || a.k_row_stride != a.v_row_stride)) return;
+    const __amdgpu_buffer_rsrc_t kr = slice_rsrc(kh, kspan);
+    const __amdgpu_buffer_rsrc_t vr = slice_rsrc(vh, vspan);
     float *obase = a.o + (size_t)head * a.o_stride;
     const size_t ors = a.o_row_stride;
 
@@ -801,7 +836,35 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // into an LDS tile (1 KB per wave-instruction, same swizzle as K) and read by every wave after
     // one barrier, instead of each wave fetching its group's rows from L2.
     half8 qf[D / 16];
-    if constexpr (XS) {
+    // UN: Q by plain loads at whatever alignment, once per workgroup, each 16-byte chunk (positions 8ch ..
+    // 8ch+7 of a row, rotated like K's) issued here and put right after the prologue's ring loads are
+    // in flight (q_fix). Rows past seq_len re-read the last (their results are dropped).
+    constexpr int NQR = !UN ? 1 : C::QLDS ? (C::BM * C::CH + C::NT - 1) / C::NT : D / 16;  // chunks per lane
+    u32x4 qraw[NQR];
+    uint32_t qlast[NQR];  // column D - 1, for chunk 0 of a rotated row
+    auto q_at = [&](int i, int &row, int &ch) {  // chunk i of this lane, and whether it has one
+        const int u = C::QLDS ? tid + C::NT * i : (32 * qg + c) * C::CH + 2 * i + hh;
+        row = u / C::CH;
+        ch = u % C::CH;
+        return u < C::BM * C::CH;
+    };
+    auto q_fix = [&](int i, int ch) {
+        const u32x4 x = qraw[i];
+        if (!kodd || ch > 0) return x;
+        return u32x4{x[0] << 16 | qlast[i], __builtin_amdgcn_alignbyte(x[1], x[0], 2),
+                     __builtin_amdgcn_alignbyte(x[2], x[1], 2), __builtin_amdgcn_alignbyte(x[3], x[2], 2)};
+    };
+    if constexpr (UN) {
+        const uint16_t *qh = a.q + (size_t)head * a.q_stride;
+#pragma unroll
+        for (int i = 0; i < NQR; ++i) {
+            int row, ch;
+            if (!q_at(i, row, ch)) continue;
+            const uint16_t *p = qh + (size_t)min(q0 + row, S - 1) * a.q_row_stride;
+            qraw[i] = load8<false>(p + (kodd && ch > 0 ? 8 * ch - 1 : 8 * ch));
+            qlast[i] = kodd ? p[D - 1] : 0u;
+        }
+    } else if constexpr (XS) {
         // Waves 0-3 stage block q's (or the solo block's) 32 rows, waves 4-7 block p's (B only).
         static_assert(C::QLOADS == 4, "one 32-row Q tile is four wave-instructions");
         const int qb_tile = (w < 4 || xs_role != 1) ? (xs_role == 1 ? xs_q : qblk) : xs_p;
@@ -855,6 +918,43 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // First key of the wave's slice in step blk (private staging): key tile tfirst + tsin + tg*blk.
     auto wave_key0 = [&](int blk) { return 32 * (tfirst + tsin + tg * blk); };
 
+    // UN: column D - 1 of the rows whose chunks this wave loads, for an odd slice: lane i holds row i of
+    // the wave's rows of K and of V (the same ones, but for a wave that stages only one of the two).
+    // A wave alone on its SIMD issues a VALU instruction every ~8 cycles, so what a step adds is kept to
+    // the loads, one offset add each, and the writes.
+    constexpr int NKV = C::LPW > 1 ? C::LPW / 2 : 1;  // the wave's instructions per tensor and block
+    constexpr int ROWS = NKV * 64 / C::CH;            // its rows
+    static_assert(!UN || ROWS <= 64, "one lane per row");
+    const int eri = lane / (64 / C::CH) % NKV, erl = lane % (64 / C::CH);  // lane's instruction and row in it
+    const int erow = erl + 64 / C::CH * (PRIV ? s * NKV + eri : C::LPW == 1 ? w % (C::LOADS / 2) : w + C::NW * eri);
+    const bool on_k = C::LPW > 1 || w < C::LOADS / 2, on_v = C::LPW > 1 || w >= C::LOADS / 2;
+    const uint32_t edge_at = (uint32_t)(uintptr_t)smem + SW::slot(erow, 0) * 16;
+    const __amdgpu_buffer_rsrc_t ker = edge_rsrc(kh, kspan), ver = edge_rsrc(vh, vspan);
+    const uint32_t eoff = (uint32_t)erow * krb + 2u * D;
+    auto key0_of = [&](int blk) { return PRIV ? wave_key0(blk) - C::WK * s : blk * C::BN; };
+    uint32_t edge_k = 0, edge_v = 0;
+    auto load_edge = [&](int blk) {
+        if (kodd && on_k) {
+            if (lane < ROWS) edge_k = __builtin_amdgcn_raw_buffer_load_b16(ker, eoff + (uint32_t)key0_of(blk) * krb, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+        if (vodd && on_v) {
+            if (lane < ROWS) edge_v = __builtin_amdgcn_raw_buffer_load_b16(ver, eoff + (uint32_t)key0_of(blk) * krb, 0, 0);
+        }
+    };
+    // Waits for the wave's loads of the block and puts the columns.
+    auto land = [&](auto stage_c) {
+        constexpr int ST = decltype(stage_c)::value * C::STAGE;
+        wait_vm_only<0>();
+        if (kodd && on_k) {
+            if (lane < ROWS) *(NC_LDS(uint16_t) *)(uintptr_t)(edge_at + ST) = (uint16_t)edge_k;
+        }
+        if (vodd && on_v) {
+            if (lane < ROWS) *(NC_LDS(uint16_t) *)(uintptr_t)(edge_at + ST + C::TILE) = (uint16_t)edge_v;
+        }
+        asm volatile("" ::: "memory");
+    };
+
     // Staging: wave-instruction t of a block fills 16-byte slots [64t, 64t+64) of the K tile
     // (t < LOADS/2) or of the V tile; the ring stage is a compile-time constant.
     auto issue = [&](int blk, auto stage_c) {
@@ -874,11 +974,13 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
             // private staging: row r of the stage is row r - 32s of the wave's 32-key slice
             const uint32_t key = PRIV ? (uint32_t)(wave_key0(blk) + r - C::WK * s) : (uint32_t)(blk * C::BN + r);
             NC_LDS(void) *dst = (NC_LDS(void) *)(sbase + (isv ? C::TILE : 0) + tt * 1024);
-            if (isv)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, dst, 16, key * vrb + ch * 16, 0, 0, 0);
-            else
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, dst, 16, key * krb + ch * 16, 0, 0, 0);
+            uint32_t off = key * (isv ? vrb : krb) + ch * 16;
+            if constexpr (UN)  // & ~3 (whole dwords already) keeps the lane's part one register across blocks
+                off = (uint32_t)key0_of(blk) * (isv ? vrb : krb) +
+                      (((uint32_t)r * (isv ? vrb : krb) + ch * 16) & ~3u);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(isv ? vr : kr, dst, 16, off, 0, 0, 0);
         }
+        if constexpr (UN) load_edge(blk);
     };
 
     // Lane-dependent LDS byte offsets of the MFMA operand reads within stage 0; stages, sub-tiles
@@ -1048,7 +1150,10 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
             }
         if constexpr (KPF) {
             if (has_next) {
-                wait_vm_only<0>();  // the wave's slice of the next block has landed
+                if constexpr (UN)
+                    land(IC<NEXT / C::STAGE>{});
+                else
+                    wait_vm_only<0>();  // the wave's slice of the next block has landed
 #pragma unroll
                 for (int kk = 0; kk < D / 16; ++kk) kpf[kk] = lds_load_b128<NEXT>(kaddr[kk]);
             }
@@ -1078,7 +1183,10 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
             // Private single stage: the wave's reads of the previous block are complete (their
             // results were consumed), so it refills the stage with this block and waits for it.
             if (blk > 0) issue(blk, IC<0>{});
-            wait_vm_only<0>();
+            if constexpr (UN)
+                land(IC<0>{});
+            else
+                wait_vm_only<0>();
         } else if constexpr (KPF) {
             // this block's slice was waited for before its K was prefetched
             if (blk + 1 < nblk) issue(blk + 1, IC<(ST + 1) % 2>{});
@@ -1093,6 +1201,11 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
                 issue(blk, IC<0>{});
             }
             wait_vm_barrier<0>();
+        } else if constexpr (UN) {
+            static_assert(NSTAGE == 2, "one block's edge column in flight");
+            land(IC<ST>{});
+            wait_vm_barrier<0>();
+            if (blk + 1 < nblk) issue(blk + 1, IC<(ST + 1) % 2>{});
         } else {
             wait_block<C::LPW, NSTAGE - 2>(min(NSTAGE - 2, nblk - 1 - blk));
             if (blk + NSTAGE - 1 < nblk) issue(blk + NSTAGE - 1, IC<(ST + NSTAGE - 1) % NSTAGE>{});
@@ -1121,7 +1234,19 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
         constexpr int I = decltype(ic)::value;
         if (!C::QLDS || I < nblk) issue(I, IC<I>{});
     });
-    if constexpr (C::QLDS)
+    if constexpr (UN) {
+#pragma unroll
+        for (int i = 0; i < NQR; ++i) {
+            int row, ch;
+            if (!q_at(i, row, ch)) continue;
+            const u32x4 x = q_fix(i, ch);
+            if constexpr (C::QLDS)
+                *(NC_LDS(u32x4) *)(uintptr_t)(lds0 + C::Q_OFF + SW::slot(row, ch) * 16) = x;
+            else
+                qf[i] = __builtin_bit_cast(half8, x);
+        }
+        wait_vm_only<0>();  // (and this wave's part of the Q tile is written)
+    } else if constexpr (C::QLDS)
         with_clamped<0, (NSTAGE > 1 ? NSTAGE - 1 : 1)>(nblk, [&](auto ac) { wait_vm_only<decltype(ac)::value * C::LPW>(); });
     else
         wait_vm_only<(NSTAGE > 1 ? NSTAGE - 1 : 1) * C::LPW>();
@@ -1135,7 +1260,10 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     use_now(qf);
     if constexpr (KPF) {
         if (nblk > 0) {
-            wait_vm_only<0>();  // block 0's slice
+            if constexpr (UN)
+                land(IC<0>{});
+            else
+                wait_vm_only<0>();  // block 0's slice
 #pragma unroll
             for (int kk = 0; kk < D / 16; ++kk) kpf[kk] = lds_load_b128<0>(kaddr[kk]);
         }
@@ -1155,6 +1283,24 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
 
     NC_TL_STAMP(tl_loop1)
     constexpr int DC = D / 4;
+    // Positions 4ch .. 4ch+3 of an output row, in lane ch of the row's DC lanes. UN with a rotated V:
+    // position e is column e - 1 (position 0 column D - 1), so lane ch's fourth column is the first
+    // position of the next of the row's lanes.
+    auto store_cols = [&](int row, int ch, floatx4 x) {
+        if constexpr (UN) {
+            float next;
+            if constexpr (DC == 16) {
+                next = dpp_f32<0x12F>(x[0]);  // row_ror:15
+            } else if constexpr (DC == 8) {
+                const float up = dpp_f32<0x101>(x[0]), wrap = dpp_f32<0x117>(x[0]);  // row_shl:1, row_shr:7
+                next = ch == DC - 1 ? wrap : up;
+            } else {
+                next = dpp_f32<0x39>(x[0]);  // quad_perm [1,2,3,0]
+            }
+            if (vodd) x = floatx4{x[1], x[2], x[3], next};
+        }
+        store_o(reinterpret_cast<floatx4 *>(obase + (size_t)row * ors + 4 * ch), x);
+    };
     float2v *mlb = reinterpret_cast<float2v *>(smem + C::ML_OFF);  // [BM queries][NS splits]
     const float lt = pair_sum(l);
     if constexpr (PRIV && NS > 1) {
@@ -1304,7 +1450,7 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
                 res += dpp_f32<0x150 + J>(wn) * pj[J];  // row_newbcast:J
             });
             const int row = q0 + qi;
-            if (row < S) store_o(reinterpret_cast<floatx4 *>(obase + (size_t)row * ors + 4 * ch), res);
+            if (row < S) store_cols(row, ch, res);
             NC_TL_END()
             return;
         }
@@ -1330,7 +1476,7 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
                 den = __builtin_fmaf(wj, ml[j][1], den);
                 res += wj * pj[j];
             }
-            store_o(reinterpret_cast<floatx4 *>(obase + (size_t)row * ors + 4 * ch), res * __builtin_amdgcn_rcpf(den));
+            store_cols(row, ch, res * __builtin_amdgcn_rcpf(den));
         }
         NC_TL_END()
         return;
@@ -1388,16 +1534,16 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
         floatx4 res = parts[0];
 #pragma unroll
         for (int j = 1; j < NS; ++j) res += parts[j];
-        store_o(reinterpret_cast<floatx4 *>(obase + (size_t)row * ors + 4 * ch), res);
+        store_cols(row, ch, res);
     }
     NC_TL_END()
 }
 
 // A dispatched pipelined kernel: its LDS, and launch index blockIdx.x mapped by pipe_slot.
-template <int D, int NQ, int NS, bool CAUSAL, int NSTAGE, int SUB, bool BF, bool XS = false>
+template <int D, int NQ, int NS, bool CAUSAL, int NSTAGE, int SUB, bool BF, bool XS = false, bool UN = false>
 __device__ __forceinline__ void flash_fwd_pipe_kernel(const nc_flash_kernel_args &a) {
     __shared__ __attribute__((aligned(16))) char smem[pipe_lds_bytes<D, NQ, NS, NSTAGE, SUB, XS>()];
-    flash_fwd_pipe_body<D, NQ, NS, CAUSAL, NSTAGE, SUB, BF, XS>(a, smem, [](uint32_t bh) { return pipe_slot(blockIdx.x, bh); });
+    flash_fwd_pipe_body<D, NQ, NS, CAUSAL, NSTAGE, SUB, BF, XS, UN>(a, smem, [](uint32_t bh) { return pipe_slot(blockIdx.x, bh); });
 }
 
 // Dense-layout form of the private-staging kernels (the `d` kernels, e.g. q1s8p2d), for launches whose four
@@ -2058,6 +2204,42 @@ NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_full, 64, 2, 4, false, 2, 1)
 NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_causal, 64, 2, 4, true, 2, 1)
 NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_full, 64, 1, 8, false, 2, 1)
 NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_causal, 64, 1, 8, true, 2, 1)
+// Slices at any 2-byte alignment (UN), with registers held to WPE waves per SIMD.
+#define NC_FLASH_UNALIGNED_PIPE_KERNEL(NAME, D, NQ, NS, CAUSAL, NSTAGE, SUB, WPE)                        \
+    extern "C" __global__ __launch_bounds__(NQ * NS * 64) __attribute__((amdgpu_waves_per_eu(WPE)))     \
+    void NAME(nc_flash_kernel_args a) {                                                                 \
+        flash_fwd_pipe_kernel<D, NQ, NS, CAUSAL, NSTAGE, SUB, false, false, true>(a);                     \
+    }                                                                                                   \
+    extern "C" __global__ __launch_bounds__(NQ * NS * 64) __attribute__((amdgpu_waves_per_eu(WPE)))     \
+    void NAME##_bf16(nc_flash_kernel_args a) {                                                          \
+        flash_fwd_pipe_kernel<D, NQ, NS, CAUSAL, NSTAGE, SUB, true, false, true>(a);                      \
+    }
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q8s1p2t2_full_unaligned, 64, 8, 1, false, 2, 2, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q8s1p2t2_causal_unaligned, 64, 8, 1, true, 2, 2, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q4s1p2t2_full_unaligned, 64, 4, 1, false, 2, 2, 3)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q4s1p2t2_causal_unaligned, 64, 4, 1, true, 2, 2, 3)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_full_unaligned, 64, 2, 4, false, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_causal_unaligned, 64, 2, 4, true, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_full_unaligned, 64, 1, 8, false, 2, 1, 2)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_causal_unaligned, 64, 1, 8, true, 2, 1, 2)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p1_full_unaligned, 64, 1, 8, false, 1, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p1_causal_unaligned, 64, 1, 8, true, 1, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q4s1p2_full_unaligned, 32, 4, 1, false, 2, 1, 5)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q4s1p2_causal_unaligned, 32, 4, 1, true, 2, 1, 5)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s4p2_full_unaligned, 32, 2, 4, false, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s4p2_causal_unaligned, 32, 2, 4, true, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p2_full_unaligned, 32, 1, 8, false, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p2_causal_unaligned, 32, 1, 8, true, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p1_full_unaligned, 32, 1, 8, false, 1, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p1_causal_unaligned, 32, 1, 8, true, 1, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q4s1p2t2_full_unaligned, 16, 4, 1, false, 2, 2, 5)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q4s1p2t2_causal_unaligned, 16, 4, 1, true, 2, 2, 5)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s4p2_full_unaligned, 16, 2, 4, false, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s4p2_causal_unaligned, 16, 2, 4, true, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q1s8p2_full_unaligned, 16, 1, 8, false, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q1s8p2_causal_unaligned, 16, 1, 8, true, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q1s8p1_full_unaligned, 16, 1, 8, false, 1, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q1s8p1_causal_unaligned, 16, 1, 8, true, 1, 1, 4)
 // Pair split (x): causal query blocks p and nqb-1-p shared by two workgroups that exchange partials.
 #define NC_FLASH_XS_KERNEL(NAME, D)                                                                     \
     extern "C" __global__ __launch_bounds__(512) void NAME(nc_flash_kernel_args a) {                     \

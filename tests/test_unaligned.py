@@ -1,0 +1,72 @@
+"""Dispatch of slices that are not 16-byte aligned (no GPU): the pipelined kernels take every layout
+whose Q/K/V rows start at dwords, their `_unaligned` forms any 2-byte alignment with one even row
+stride for K and V, and the generic kernels the rest."""
+
+import itertools
+
+import pytest
+
+import notcute_flash as nc
+
+BASE = 1 << 20
+
+
+def route(bh, s, d, causal, q=BASE, k=BASE, v=BASE, o=BASE, rows=(0, 0, 0, 0), pads=(0, 0, 0, 0), dtype="f16"):
+    r = [x or d for x in rows]
+    opts = nc.options(batch_heads=bh, seq_len=s, head_dim=d, causal=causal, dtype=dtype, q_row_stride=rows[0],
+                      k_row_stride=rows[1], v_row_stride=rows[2], o_row_stride=rows[3], q_stride=s * r[0] + pads[0],
+                      k_stride=s * r[1] + pads[1], v_stride=s * r[2] + pads[2], o_stride=s * r[3] + pads[3])
+    sel = nc.select_kernel_for(opts, q, k, v, o)
+    name = sel.name.decode()
+    family = "generic" if "_m64_" in name else "unaligned" if "_unaligned" in name else "pipe"
+    return family, sel
+
+
+SHAPES = [(1, 1, 16), (3, 49, 16), (8, 250, 32), (8, 1024, 64), (16, 1500, 64), (64, 2048, 16), (128, 1000, 32),
+          (64, 512, 64), (4, 8192, 64), (32, 4096, 64)]
+
+
+@pytest.mark.parametrize("bh,s,d", SHAPES)
+@pytest.mark.parametrize("causal", [False, True])
+def test_route_follows_the_layout(bh, s, d, causal):
+    for offs in itertools.product((0, 1, 2, 4), repeat=3):  # elements past 16-byte alignment of Q, K, V
+        ptr = dict(zip("qkv", (BASE + 2 * x for x in offs)))
+        family, sel = route(bh, s, d, causal, **ptr)
+        assert family == ("unaligned" if 1 in offs else "pipe"), offs
+        assert sel.aligned == (1 if not any(offs) else 0)
+    for pads in itertools.product((0, 3, 6), repeat=3):
+        family, sel = route(bh, s, d, causal, pads=pads + (5,))
+        assert family == ("unaligned" if 3 in pads else "pipe"), pads
+        assert sel.aligned == 0
+    # O: any float; an address between floats, and odd, differing or odd-element K/V rows: generic
+    assert route(bh, s, d, causal, o=BASE + 4)[0] == "pipe"
+    assert route(bh, s, d, causal, o=BASE + 2)[0] == "generic"
+    assert route(bh, s, d, causal, q=BASE + 1)[0] == "generic"
+    assert route(bh, s, d, causal, rows=(d + 2, d + 2, d + 4, d + 1))[0] == "pipe"
+    assert route(bh, s, d, causal, rows=(d + 1, d + 2, d + 2, 0))[0] == "unaligned"
+    assert route(bh, s, d, causal, k=BASE + 2, rows=(0, d + 2, d + 4, 0))[0] == "generic"
+    assert route(bh, s, d, causal, rows=(0, d + 1, d + 1, 0))[0] == "generic"
+
+
+@pytest.mark.parametrize("bh,s,d", SHAPES)
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_unaligned_selection_is_launchable(bh, s, d, dtype):
+    for causal in (False, True):
+        _, al = route(bh, s, d, causal, dtype=dtype)
+        _, un = route(bh, s, d, causal, k=BASE + 2, dtype=dtype)
+        assert un.name.decode().endswith("_unaligned_bf16" if dtype == "bf16" else "_unaligned")
+        assert un.block_m == al.block_m and un.threads == al.threads and un.scratch_bytes == 0
+        assert un.grid[0] == -(-s // un.block_m) * bh and un.grid[1] == un.grid[2] == 1
+
+
+def test_no_new_scratch_and_no_new_refusals():
+    """The pair split's scratch stays with 16-byte aligned slices, and a grid that only the generic
+    kernels' workgroups fit keeps them."""
+    assert route(1, 4096, 64, True)[1].scratch_bytes > 0
+    for ptr in (BASE + 4, BASE + 2):
+        assert route(1, 4096, 64, True, q=ptr)[1].scratch_bytes == 0
+    for d in (16, 32, 64):
+        for ptr in (BASE + 4, BASE + 2):
+            family, sel = route((1 << 23) - 1, 1, d, False, q=ptr)
+            assert sel.grid[0] * sel.threads <= 0xFFFFFFFF
+    assert route((1 << 24) - 1, 1, 32, False, q=BASE + 2)[1].threads == 256

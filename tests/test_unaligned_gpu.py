@@ -1,0 +1,107 @@
+"""The `_unaligned` pipelined kernels against the oracle: every kernel by name, every combination of
+odd and even Q/K/V slices at tile edges, with infinities and NaNs in everything around the slices
+(a neighbouring element that reached a product would show), and the dword-aligned layouts that the
+plain pipelined kernels take."""
+
+import itertools
+import math
+import os
+import re
+
+import numpy as np
+import pytest
+
+import flashcheck as fc
+import notcute_flash as nc
+from flash_workloads import Workload
+
+pytestmark = pytest.mark.gpu
+
+POISON = {"f16": np.array([0x7C00, 0x7E00, 0xFC00], np.uint16), "bf16": np.array([0x7F80, 0x7FC0, 0xFF80], np.uint16)}
+
+
+def poisoned(wl: Workload, arr, which, offset):
+    """The tensor in a buffer `offset` elements longer, all that is not an active element poisoned."""
+    out = np.resize(POISON[wl.dtype], arr.size + offset + 8)
+    b = np.arange(wl.batch_heads)[:, None, None] * wl.stride(which)
+    idx = (b + np.arange(wl.seq_len)[None, :, None] * wl.row(which) + np.arange(wl.head_dim)).reshape(-1)
+    out[idx + offset] = arr[idx]
+    return out
+
+
+def check(gpu, wl, offs, name=None):
+    print(f"[case] {wl.describe()} {wl.dtype} offsets={offs} {name or ''}", flush=True)
+    tensors = wl.make_inputs()
+    o_init = np.full(wl.length("o"), fc.SENTINEL, dtype=np.float32)
+    ref = fc.oracle(wl, *tensors, o_init=o_init)
+    bufs = [nc.DeviceBuffer.from_array(poisoned(wl, t, w, f)) for t, w, f in zip(tensors, "qkv", offs)]
+    bufs.append(nc.DeviceBuffer.from_array(o_init))
+    try:
+        ptr = [b.ptr + 2 * f for b, f in zip(bufs, offs)] + [bufs[3].ptr]
+        sel = nc.select_kernel_for(wl.options(), *ptr)
+        if name is None:
+            name, grid, threads = sel.name.decode(), tuple(sel.grid), sel.threads
+        else:
+            m = re.search(r"_q(\d+)s(\d+)p", name)
+            sel = nc.KernelSelection()
+            sel.block_m, threads = 32 * int(m.group(1)), 64 * int(m.group(1)) * int(m.group(2))
+            grid = (-(-wl.seq_len // sel.block_m) * wl.batch_heads,)
+        args = nc.pack_args(wl.options(), sel, *ptr)
+        gpu.get_function(name).launch(grid, (threads,), nc.kernel_params(name, args))
+        nc.synchronize()
+        out = bufs[3].download(np.float32, wl.length("o"))
+    finally:
+        for b in bufs:
+            b.free()
+    # the parity bar of the element type (f16 2e-3 / 1e-2, bf16 8e-3 / 4e-2): the same arithmetic as the
+    # aligned kernels, in another order over the head columns
+    max_abs, max_rel = fc.parity_bar(wl.dtype)
+    fc.assert_parity(out, ref, fc.active_index(wl), name, max_abs=max_abs, max_rel=max_rel)
+    fc.assert_pads_untouched(out, o_init, wl, name)
+    return name
+
+
+def _names():
+    src = open(os.path.join(os.path.dirname(__file__), "..", "not-cute-zig_amd", "csrc", "flash_fwd.hip")).read()
+    names = re.findall(r"NC_FLASH_UNALIGNED_PIPE_KERNEL\((nc_flash_fwd_\w+),", src)
+    return sorted(n + t for n in names for t in ("", "_bf16"))
+
+
+@pytest.mark.parametrize("name", _names())
+def test_each_unaligned_kernel(gpu, name):
+    """S = 1100: several blocks per wave in every kernel, no multiple of any tile. Three slices whose
+    strides make Q, K, V even and odd in turn; no kernel may use scratch."""
+    d = int(re.search(r"_d(\d+)_", name).group(1))
+    assert gpu.get_function(name).attributes().local_size_bytes == 0
+    s = 1100
+    wl = Workload(f"un_{name}", 3, s, d, "_causal" in name, 1.0 / math.sqrt(d), (("normal", 0.0, 1.0),) * 3, seed=31,
+                  q_stride=s * d + 17, k_stride=s * d + 19, v_stride=s * d + 23, o_stride=s * d + 29,
+                  dtype="bf16" if name.endswith("_bf16") else "f16")
+    check(gpu, wl, (0, 1, 0), name)
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("causal", [False, True])
+def test_phases_and_lengths(gpu, d, causal):
+    """Every combination of odd and even Q, K, V at the lengths around the tiles and blocks, packed and
+    padded rows (an odd Q pitch among them)."""
+    for i, s in enumerate((1, 2, 31, 32, 33, 64, 65, 127, 128, 129, 257, 513)):
+        row = {} if i % 3 else dict(q_row=d + 5, k_row=d + 6, v_row=d + 6, o_row=d + 3)
+        for offs in itertools.product((0, 1), repeat=3):
+            wl = Workload(f"ph{s}", 2, s, d, causal, (-0.3 if i % 4 == 3 else 1.0 / math.sqrt(d)),
+                          (("normal", 0.0, 1.0),) * 3, seed=40 + i, o_stride=s * (d + 3) + 1, **row)
+            check(gpu, wl, offs)
+
+
+@pytest.mark.parametrize("bh,s,d,causal", [(8, 250, 32, True), (96, 333, 64, True), (24, 1500, 64, False),
+                                           (128, 700, 16, False), (3, 3100, 64, True), (96, 130, 32, False)])
+@pytest.mark.parametrize("offs", [(2, 4, 6), (1, 2, 4), (0, 3, 0), (0, 0, 5)])
+def test_dispatched_routes(gpu, bh, s, d, causal, offs):
+    """Through the selection: dword-aligned slices on the plain pipelined kernels (causal BH=3 S=3100
+    would take the pair split if it were 16-byte aligned), odd ones on the `_unaligned` kernels."""
+    wl = Workload(f"route_{bh}_{s}_{d}", bh, s, d, causal, 1.0 / math.sqrt(d), (("normal", 0.0, 1.0),) * 3, seed=50)
+    opts = wl.options()
+    sel = nc.select_kernel_for(opts, *[(1 << 20) + 2 * f for f in offs], 1 << 20)
+    assert sel.name.decode().endswith("_unaligned") == any(f % 2 for f in offs)
+    assert sel.scratch_bytes == 0
+    check(gpu, wl, offs)
