@@ -77,6 +77,14 @@ __device__ __forceinline__ floatx16 mfma32(half8 a, half8 b, floatx16 c) {
     else
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
+template <bool BF>
+__device__ __forceinline__ floatx4 mfma16(half8 a, half8 b, floatx4 c) {
+    if constexpr (BF)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                       0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
 // Two weights rounded (to nearest even) to the element type, packed as one dword.
 template <bool BF>
 __device__ __forceinline__ half2v round2(float x, float y) {
@@ -918,6 +926,9 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // First key of the wave's slice in step blk (private staging): key tile tfirst + tsin + tg*blk.
     auto wave_key0 = [&](int blk) { return 32 * (tfirst + tsin + tg * blk); };
 
+    // Key of row 0 of a block's stage, as this wave's rows see it.
+    auto key0_of = [&](int blk) { return PRIV ? wave_key0(blk) - C::WK * s : blk * C::BN; };
+
     // UN: column D - 1 of the rows whose chunks this wave loads, for an odd slice: lane i holds row i of
     // the wave's rows of K and of V (the same ones, but for a wave that stages only one of the two).
     // A wave alone on its SIMD issues a VALU instruction every ~8 cycles, so what a step adds is kept to
@@ -931,7 +942,6 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     const uint32_t edge_at = (uint32_t)(uintptr_t)smem + SW::slot(erow, 0) * 16;
     const __amdgpu_buffer_rsrc_t ker = edge_rsrc(kh, kspan), ver = edge_rsrc(vh, vspan);
     const uint32_t eoff = (uint32_t)erow * krb + 2u * D;
-    auto key0_of = [&](int blk) { return PRIV ? wave_key0(blk) - C::WK * s : blk * C::BN; };
     uint32_t edge_k = 0, edge_v = 0;
     auto load_edge = [&](int blk) {
         if (kodd && on_k) {
@@ -971,13 +981,22 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
             const int p = tt * 64 + lane;
             const int r = p / C::CH, sl = p % C::CH;
             const int ch = sl ^ SW::f(r);
-            // private staging: row r of the stage is row r - 32s of the wave's 32-key slice
-            const uint32_t key = PRIV ? (uint32_t)(wave_key0(blk) + r - C::WK * s) : (uint32_t)(blk * C::BN + r);
             NC_LDS(void) *dst = (NC_LDS(void) *)(sbase + (isv ? C::TILE : 0) + tt * 1024);
-            uint32_t off = key * (isv ? vrb : krb) + ch * 16;
-            if constexpr (UN)  // & ~3 (whole dwords already) keeps the lane's part one register across blocks
-                off = (uint32_t)key0_of(blk) * (isv ? vrb : krb) +
-                      (((uint32_t)r * (isv ? vrb : krb) + ch * 16) & ~3u);
+            const uint32_t rb = isv ? vrb : krb;
+            uint32_t off;
+            if constexpr (!PRIV) {
+                // A scalar part per block and instruction plus a lane part per tensor (the swizzle repeats
+                // every 16 rows). Left to itself the compiler keeps one offset per instruction in a VGPR
+                // across the key loop: 121 against 128 and 7 spilled on the d=64 q4s1 kernel.
+                constexpr int RPI = 64 / C::CH;
+                uint32_t u = (uint32_t)(blk * C::BN + tt * RPI) * rb;
+                asm volatile("" : "+s"(u));
+                off = u + (uint32_t)(lane / C::CH) * rb + ((lane % C::CH) ^ SW::f(lane / C::CH + tt * RPI % 16)) * 16;
+            } else if constexpr (UN) {  // & ~3 (whole dwords already) keeps the lane's part one register across blocks
+                off = (uint32_t)key0_of(blk) * rb + (((uint32_t)r * rb + ch * 16) & ~3u);
+            } else {  // row r of the stage is row r - 32s of the wave's 32-key slice
+                off = (uint32_t)(wave_key0(blk) + r - C::WK * s) * rb + ch * 16;
+            }
             __builtin_amdgcn_raw_ptr_buffer_load_lds(isv ? vr : kr, dst, 16, off, 0, 0, 0);
         }
         if constexpr (UN) load_edge(blk);
@@ -1009,20 +1028,39 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // Log2-domain scale. A negative scale is applied by negating the resident Q operand (exact),
     // a zero scale by a tiny positive one (every score then rounds to weight exp2(0) = 1, as with
     // a zero scale), so the softmax below can assume sc > 0.
-    // Row sum of a tile: the weights exactly as rounded into P, added by v_dot2c against 1.0 pairs,
-    // so numerator and denominator carry the same rounding. (Dividing by the sum of the unrounded
-    // f32 weights, as the reference does, biases O by up to the rounding's relative error, 2^-11 for
-    // f16, times |V| whenever the dominant weights round the same way: 7.8e-3 at |V| = 16.)
-    // v_dot2c does not execute while an MFMA of the same SIMD is in flight (measured: 8 v_dot2c per
-    // 32x32x16 MFMA take longer than both run one after the other, where FMA, exp and the f16
-    // packing hide the MFMAs entirely), but it keeps the fewest registers live.
+    // Row sum of a tile: the weights exactly as rounded into P, so numerator and denominator carry the
+    // same rounding. (Dividing by the sum of the unrounded f32 weights, as the reference does, biases
+    // O by up to the rounding's relative error, 2^-11 for f16, times |V| whenever the dominant weights
+    // round the same way: 7.8e-3 at |V| = 16.)
+    // MSUM: two 16x16x32 MFMAs against a pattern of ones and zeros. Read as that shape's B operand, a
+    // P register holds queries n (k-groups 0, 2) and n + 16 (k-groups 1, 3) in column n, and lane l's
+    // four results are rows 4(l/16) ..: ones where (row/4) % 2 == k-group % 2 give every lane the sum
+    // of its own query's 32 weights. 32 matrix-core cycles per tile in place of 8 v_dot2c, which do not
+    // execute while an MFMA of the same SIMD is in flight (~10 cycles each). The zeros are no barrier
+    // to a weight that overflowed or is NaN, so such a tile's sums are not used: its redo adds each
+    // lane's own weights by v_dot2c. The private-staging kernels of d = 32 and 64, whose few waves wait
+    // on the tile's serial chain (S^T, weights, sum, PV), lose by the longer one (c3 5.59 -> 5.87 us), and
+    // the odd-slice q8s1 kernel has no registers for it: v_dot2c there.
+    // Measured against v_dot2c (with the first tile's max and one check per tile below): BH=32 S=4096
+    // d=64 146.9 -> 139.8 us, BH=64 S=4096 d=64 causal 156.6 -> 146.2, BH=128 S=512 d=64 causal 11.85 ->
+    // 10.97, BH=4 S=8192 d=64 causal 54.9 -> 50.9, BH=32 S=4096 d=32 104.8 -> 101.8, BH=64 S=2048 d=16
+    // 48.8 -> 45.7.
+    constexpr bool MSUM = D == 16 || (!PRIV && !(UN && NQ == 8));
+    u32x4 ones = {0u, 0u, 0u, 0u};
+    if (MSUM && ((lane >> 2) & 1) == ((lane >> 4) & 1)) {
+        const uint32_t one2 = BF ? 0x3f803f80u : 0x3c003c00u;
+        ones = u32x4{one2, one2, one2, one2};
+    }
     float sc = a.scale * kLog2e;
     const bool neg_q = sc < 0.f;  // Q is negated once it has landed
     if (neg_q) sc = -sc;
     if (!(sc > 0.f) && sc == 0.f) sc = 1e-30f;
-    float mrow = neg_inf();  // running max of sc * score (log2 domain); -inf: none yet
-    float neg_m = 0.f;       // -mrow, 0 while mrow is -inf
-    float l = 0.f;
+    if constexpr (MSUM) sc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sc)));  // a scalar register
+    float mrow = neg_inf();  // running max of sc * score (log2 domain); -inf: none yet (MSUM: -neg_m)
+    // What the weights are formed with: -mrow; while mrow is -inf, 0, or with MSUM +inf, so that the
+    // first tile a row sees overflows and takes its max without a test of its own.
+    float neg_m = MSUM ? __builtin_inff() : 0.f;
+    float l = 0.f;  // row sum: this lane's keys, with MSUM all of the wave's
     floatx16 o[C::MT];
 #pragma unroll
     for (int mt = 0; mt < C::MT; ++mt) o[mt] = floatx16{};
@@ -1037,7 +1075,8 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // One 32x32 sub-tile of this wave: S^T = K Q^T for its 32 keys (kt0 ..), online softmax, and
     // O^T += V^T P^T. TOFF is the sub-tile's byte offset in the LDS ring (a compile-time constant);
     // with K prefetch, NEXT is the next tile's offset and has_next says whether the wave has one.
-    auto tile = [&](const int kt0, auto toff_c, auto next_c, const bool has_next) {
+    // first: no tile of the wave has been taken yet.
+    auto tile = [&](const int kt0, auto toff_c, auto next_c, const bool has_next, const bool first) {
         constexpr int TOFF = decltype(toff_c)::value;
         constexpr int NEXT = decltype(next_c)::value;
 
@@ -1091,34 +1130,51 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
             }
         }
         half8 pf[2];
-        auto weights = [&]() {
-            {
-                float ls = 0.f;
+        // P of the tile and its row sum (the lane's own keys; on the matrix cores, all of the wave's).
+        auto weights = [&](auto mfma_c) {
+            constexpr bool MF = decltype(mfma_c)::value != 0;
+            float ls = 0.f;
 #pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
-                    half2v h[4];
+            for (int ks = 0; ks < 2; ++ks) {
+                half2v h[4];
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        h[t] = round2<BF>(__builtin_amdgcn_exp2f(__builtin_fmaf(acc[8 * ks + 2 * t], sc, neg_m)),
-                                          __builtin_amdgcn_exp2f(__builtin_fmaf(acc[8 * ks + 2 * t + 1], sc, neg_m)));
-                        pf[ks][2 * t] = h[t][0];
-                        pf[ks][2 * t + 1] = h[t][1];
-                    }
+                for (int t = 0; t < 4; ++t) {
+                    h[t] = round2<BF>(__builtin_amdgcn_exp2f(__builtin_fmaf(acc[8 * ks + 2 * t], sc, neg_m)),
+                                      __builtin_amdgcn_exp2f(__builtin_fmaf(acc[8 * ks + 2 * t + 1], sc, neg_m)));
+                    pf[ks][2 * t] = h[t][0];
+                    pf[ks][2 * t + 1] = h[t][1];
+                }
+                if constexpr (!MF) {
 #pragma unroll
                     for (int t = 0; t < 4; ++t) ls = sum2<BF>(h[t], ls);
                 }
-                return ls;
             }
+            if constexpr (MF) {
+                floatx4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) z = mfma16<BF>(__builtin_bit_cast(half8, ones), pf[ks], z);
+                ls = z[0];
+            }
+            return ls;
         };
         // Move the running max to the tile max (rows whose max does not grow keep it) and rescale.
         auto to_tile_max = [&]() {
             const floatx16 &x = acc;
-            const float m0 = fmaxf(fmaxf(x[0], x[1]), x[2]), m1 = fmaxf(fmaxf(x[3], x[4]), x[5]);
-            const float m2 = fmaxf(fmaxf(x[6], x[7]), x[8]), m3 = fmaxf(fmaxf(x[9], x[10]), x[11]);
-            const float m4 = fmaxf(fmaxf(x[12], x[13]), x[14]);
-            // (folding -inf in first lets the compiler fuse the tree into v_max3 without extra
-            // canonicalising maxes)
-            const float tmax = fmaxf(neg_inf(), fmaxf(fmaxf(fmaxf(m0, m1), m2), fmaxf(fmaxf(m3, m4), x[15])));
+            float tmax;
+            if constexpr (MSUM) {
+                tmax = neg_inf();
+                asm volatile("" : "+v"(tmax));  // or the compiler forms it beside every tile's weights
+#pragma unroll
+                for (int r = 0; r < 16; r += 2) tmax = fmaxf(fmaxf(tmax, x[r]), x[r + 1]);
+                mrow = -neg_m;
+            } else {
+                const float m0 = fmaxf(fmaxf(x[0], x[1]), x[2]), m1 = fmaxf(fmaxf(x[3], x[4]), x[5]);
+                const float m2 = fmaxf(fmaxf(x[6], x[7]), x[8]), m3 = fmaxf(fmaxf(x[9], x[10]), x[11]);
+                const float m4 = fmaxf(fmaxf(x[12], x[13]), x[14]);
+                // (folding -inf in first lets the compiler fuse the tree into v_max3 without extra
+                // canonicalising maxes)
+                tmax = fmaxf(neg_inf(), fmaxf(fmaxf(fmaxf(m0, m1), m2), fmaxf(fmaxf(m3, m4), x[15])));
+            }
             const float m_new = fmaxf(mrow, pair_max(tmax) * sc);
             const float alpha = __builtin_amdgcn_exp2f(mrow - (m_new == neg_inf() ? 0.f : m_new));
             l *= alpha;
@@ -1127,15 +1183,27 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
             mrow = m_new;
             neg_m = (mrow == neg_inf()) ? 0.f : -mrow;
         };
-        float ls;
-        if (__builtin_amdgcn_ballot_w64(mrow == neg_inf())) {
+        float ls = 0.f;
+        if constexpr (MSUM) {
+            // (the first tile's max is taken at once, every other one's when its sums show the need)
+            bool redo = first;
+            if (!first) {
+                ls = weights(IC<1>{});
+                redo = __builtin_amdgcn_ballot_w64(!(ls < weight_sum_limit<BF>())) != 0;
+            }
+            if (redo) {
+                to_tile_max();
+                ls = pair_sum(weights(IC<0>{}));
+                if (mrow == neg_inf()) neg_m = __builtin_inff();  // a row that has seen no key yet
+            }
+        } else if (__builtin_amdgcn_ballot_w64(mrow == neg_inf())) {
             to_tile_max();  // some row has no max yet: take it first
-            ls = weights();
+            ls = weights(IC<0>{});
         } else {
-            ls = weights();
+            ls = weights(IC<0>{});
             if (__builtin_amdgcn_ballot_w64(!(ls < weight_sum_limit<BF>()))) {
                 to_tile_max();  // a weight overflowed (f16) or grew too large (bf16): redo the tile
-                ls = weights();
+                ls = weights(IC<0>{});
             }
         }
         l += ls;
@@ -1220,7 +1288,8 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
         if (!run) return;
         static_for<0, SUB>([&](auto jc) {
             constexpr int TOFF = ST * C::STAGE + 2 * decltype(jc)::value * ROW16;  // sub-tile in the stage
-            tile(kb + 32 * decltype(jc)::value, IC<TOFF>{}, IC<((ST + 1) % NSTAGE) * C::STAGE>{}, blk + 1 < nblk);
+            tile(kb + 32 * decltype(jc)::value, IC<TOFF>{}, IC<((ST + 1) % NSTAGE) * C::STAGE>{}, blk + 1 < nblk,
+                 ST == 0 && decltype(jc)::value == 0 && blk == 0);
             __builtin_amdgcn_sched_barrier(0);  // keep sub-tiles (and steps) apart
         });
     };
@@ -1302,7 +1371,8 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
         store_o(reinterpret_cast<floatx4 *>(obase + (size_t)row * ors + 4 * ch), x);
     };
     float2v *mlb = reinterpret_cast<float2v *>(smem + C::ML_OFF);  // [BM queries][NS splits]
-    const float lt = pair_sum(l);
+    const float lt = MSUM ? l : pair_sum(l);
+    if constexpr (MSUM) mrow = -neg_m;
     if constexpr (PRIV && NS > 1) {
         // Epilogue, private staging: once a wave is past its loop, the K and V slices of ring
         // stage 0 that only it ever loaded are free, so it writes its unscaled O^T partial there
@@ -2198,10 +2268,10 @@ extern "C" __global__ __launch_bounds__(768) void nc_util_mfma_ceiling(const hal
 // Pipelined variants: q = query waves (32 rows each), s = key-split waves, p = LDS ring depth.
 NC_FLASH_PIPE_KERNEL_WPE(nc_flash_fwd_d64_q8s1p2t2_full, 64, 8, 1, false, 2, 2, 4)
 NC_FLASH_PIPE_KERNEL_WPE(nc_flash_fwd_d64_q8s1p2t2_causal, 64, 8, 1, true, 2, 2, 4)
-NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q4s1p2t2_full, 64, 4, 1, false, 2, 2)
-NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q4s1p2t2_causal, 64, 4, 1, true, 2, 2)
-NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_full, 64, 2, 4, false, 2, 1)
-NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_causal, 64, 2, 4, true, 2, 1)
+NC_FLASH_PIPE_KERNEL_WPE(nc_flash_fwd_d64_q4s1p2t2_full, 64, 4, 1, false, 2, 2, 4)
+NC_FLASH_PIPE_KERNEL_WPE(nc_flash_fwd_d64_q4s1p2t2_causal, 64, 4, 1, true, 2, 2, 4)
+NC_FLASH_PIPE_KERNEL_WPE(nc_flash_fwd_d64_q2s4p2_full, 64, 2, 4, false, 2, 1, 4)
+NC_FLASH_PIPE_KERNEL_WPE(nc_flash_fwd_d64_q2s4p2_causal, 64, 2, 4, true, 2, 1, 4)
 NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_full, 64, 1, 8, false, 2, 1)
 NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_causal, 64, 1, 8, true, 2, 1)
 // Slices at any 2-byte alignment (UN), with registers held to WPE waves per SIMD.
