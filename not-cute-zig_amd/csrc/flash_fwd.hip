@@ -643,16 +643,47 @@ struct PipeSlot {
     uint32_t L, head, qb_rev;
 };
 
+// Workgroups of a causal pipelined kernel that share a CU from the start of a launch (by its LDS and
+// registers).
+template <int D, int NQ, int NS, int NSTAGE, int SUB>
+constexpr int pipe_layers() {
+    using C = PipeCfg<D, NQ, NS, NSTAGE, SUB>;
+    constexpr int by_lds = 160 * 1024 / C::LDS_BYTES, by_regs = (D == 64 ? 4 : D == 32 || NQ == 1 ? 5 : 6) * 4 / C::NW;
+    return by_lds < by_regs ? by_lds : by_regs;
+}
+
+// Index i of n in launch order, `per` to a layer (one workgroup per CU), to its place in the order of
+// falling work: every other one of the first LAYERS layers is turned round. They all start at once, CU j
+// taking the j-th of each layer, and in plain falling order CU 0 would hold the heaviest of every
+// layer; turned, the layers' weights add up to the same on every CU, and a last, partial layer falls to
+// the CUs whose others are lightest. Later layers go to the CUs that come free, heaviest first.
+// Measured on MI355X against falling order throughout: BH=32 S=4000 d=64 causal q8s1 87.3 -> 79.5 us,
+// q4s1 82.3 -> 78.0; BH=24 S=1000 q2s4 8.76 -> 8.23; BH=64 S=2047 d=32 q4s1 30.0 -> 28.8; BH=64 S=2048 d=16
+// q4s1 26.1 -> 25.1; grids of many layers, and q2s4 where one workgroup's own keys take the whole launch
+// (BH=4 S=8192), within 1 %.
+template <int LAYERS>
+__device__ __forceinline__ uint32_t layered(uint32_t i, uint32_t n, uint32_t per) {
+    if (LAYERS < 2 || n <= per) return i;
+    const uint32_t layer = i / per;
+    if (layer >= (uint32_t)LAYERS || (layer & 1u)) return i;
+    const uint32_t base = layer * per, len = min(per, n - base);
+    return base + len - 1u - (i - base);
+}
+
 // The dispatched kernels' mapping of launch index L to its slot. Workgroups are dealt round-robin
 // to the 8 XCDs (L mod 8), so with batch_heads a multiple of 8 each XCD takes whole slices
-// (batch_heads/8 of them): every K/V slice is read through one XCD's L2. Within an XCD the query
-// blocks go heaviest (causal) first.
-__device__ __forceinline__ PipeSlot pipe_slot(uint32_t L, uint32_t bh) {
+// (batch_heads/8 of them): every K/V slice is read through one XCD's L2. Within an XCD (32 CUs) the
+// query blocks go heaviest (causal) first, by layers. Other batch_heads: over all 256 CUs, whole ranks
+// of query blocks where they fill a layer, so that a head keeps its XCDs.
+template <int LAYERS>
+__device__ __forceinline__ PipeSlot pipe_slot(uint32_t L, uint32_t bh, uint32_t nqb) {
     if ((bh & 7u) == 0) {
-        const uint32_t hpx = bh >> 3, x = L & 7u, idx = L >> 3;
+        const uint32_t hpx = bh >> 3, x = L & 7u, idx = layered<LAYERS>(L >> 3, nqb * hpx, 32u);
         return PipeSlot{L, x * hpx + idx % hpx, idx / hpx};
     }
-    return PipeSlot{L, L % bh, L / bh};
+    if (LAYERS > 1 && 256u % bh == 0) return PipeSlot{L, L % bh, layered<LAYERS>(L / bh, nqb, 256u / bh)};
+    const uint32_t M = layered<LAYERS>(L, nqb * bh, 256u);
+    return PipeSlot{L, M % bh, M / bh};
 }
 
 // LDS the pipelined body needs (the pair-split kernels add a second Q tile and the exchange words).
@@ -1613,7 +1644,10 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
 template <int D, int NQ, int NS, bool CAUSAL, int NSTAGE, int SUB, bool BF, bool XS = false, bool UN = false>
 __device__ __forceinline__ void flash_fwd_pipe_kernel(const nc_flash_kernel_args &a) {
     __shared__ __attribute__((aligned(16))) char smem[pipe_lds_bytes<D, NQ, NS, NSTAGE, SUB, XS>()];
-    flash_fwd_pipe_body<D, NQ, NS, CAUSAL, NSTAGE, SUB, BF, XS, UN>(a, smem, [](uint32_t bh) { return pipe_slot(blockIdx.x, bh); });
+    flash_fwd_pipe_body<D, NQ, NS, CAUSAL, NSTAGE, SUB, BF, XS, UN>(a, smem, [&](uint32_t bh) {
+        constexpr int LAYERS = CAUSAL && !XS ? pipe_layers<D, NQ, NS, NSTAGE, SUB>() : 1;
+        return pipe_slot<LAYERS>(blockIdx.x, bh, a.num_q_blocks);
+    });
 }
 
 // Dense-layout form of the private-staging kernels (the `d` kernels, e.g. q1s8p2d), for launches whose four
