@@ -78,11 +78,12 @@ struct Variant {
 // Two 32-key sub-tiles per wave per block ("t2": 32*NS*2 keys per block).
 #define PIPE2(D, NQ, NS, P, C, T, BF) {"nc_flash_fwd_d" #D "_q" #NQ "s" #NS "p" #P "t2_" C T, D, NQ, NS, P, 2, \
                                        C[0] == 'c', true, Family::kPipe, BF}
-// Slices at any 2-byte alignment (SUF: "" or "t2").
-#define PIPEU(D, NQ, NS, P, SUB, SUF, C, T, BF) {"nc_flash_fwd_d" #D "_q" #NQ "s" #NS "p" #P SUF "_" C "_unaligned" T, \
-                                                 D, NQ, NS, P, SUB, C[0] == 'c', false, Family::kPipe, BF}
-#define PIPEU2(D, NQ, NS, P, SUB, SUF, T, BF) PIPEU(D, NQ, NS, P, SUB, SUF, "full", T, BF), \
-    PIPEU(D, NQ, NS, P, SUB, SUF, "causal", T, BF)
+// Slices at any 2-byte alignment.
+#define PIPEU(D, NQ, NS, P, C, T, BF) {"nc_flash_fwd_d" #D "_q" #NQ "s" #NS "p" #P "_" C "_unaligned" T, \
+                                       D, NQ, NS, P, 1, C[0] == 'c', false, Family::kPipe, BF}
+#define PIPEU2(D, NQ, NS, P, T, BF) PIPEU(D, NQ, NS, P, "full", T, BF), PIPEU(D, NQ, NS, P, "causal", T, BF)
+#define PIPEU8(D, T, BF) PIPEU2(D, 2, 4, 2, T, BF), PIPEU2(D, 2, 2, 2, T, BF), PIPEU2(D, 1, 8, 2, T, BF), \
+    PIPEU2(D, 1, 8, 1, T, BF)
 #define GEN(D, C, A, SUF, T, BF) {"nc_flash_fwd_d" #D "_m64_" C SUF T, D, 2, 2, 1, 1, C[0] == 'c', A, \
                                   Family::kGeneric, BF}
 // The generic body in other geometries (32 rows x 8 key splits; 128 rows x 2 key splits).
@@ -108,11 +109,7 @@ struct Variant {
     PIPE(64, 1, 8, 1, "full", T, BF), PIPE(64, 1, 8, 1, "causal", T, BF), PIPE(32, 1, 8, 1, "full", T, BF),   \
     PIPE(32, 1, 8, 1, "causal", T, BF), PIPE(16, 1, 8, 1, "full", T, BF), PIPE(16, 1, 8, 1, "causal", T, BF), \
     PIPED4(64, T, BF), PIPED4(32, T, BF), PIPED4(16, T, BF),                                                  \
-    PIPEU2(64, 8, 1, 2, 2, "t2", T, BF), PIPEU2(64, 4, 1, 2, 2, "t2", T, BF), PIPEU2(64, 2, 4, 2, 1, "", T, BF), \
-    PIPEU2(64, 1, 8, 2, 1, "", T, BF), PIPEU2(64, 1, 8, 1, 1, "", T, BF), PIPEU2(32, 4, 1, 2, 1, "", T, BF),   \
-    PIPEU2(32, 2, 4, 2, 1, "", T, BF), PIPEU2(32, 1, 8, 2, 1, "", T, BF), PIPEU2(32, 1, 8, 1, 1, "", T, BF),   \
-    PIPEU2(16, 4, 1, 2, 2, "t2", T, BF), PIPEU2(16, 2, 4, 2, 1, "", T, BF), PIPEU2(16, 1, 8, 2, 1, "", T, BF), \
-    PIPEU2(16, 1, 8, 1, 1, "", T, BF)
+    PIPEU8(64, T, BF), PIPEU8(32, T, BF), PIPEU8(16, T, BF)
 
 const Variant kVariants[] = {VARIANTS("", false), VARIANTS("_bf16", true)};
 #undef VARIANTS
@@ -123,6 +120,7 @@ const Variant kVariants[] = {VARIANTS("", false), VARIANTS("_bf16", true)};
 #undef PIPED4
 #undef PIPEU
 #undef PIPEU2
+#undef PIPEU8
 #undef GEN
 #undef GENG
 #undef GENG2
@@ -144,11 +142,11 @@ const Variant *find_pipe_stages(uint32_t d, uint32_t nq, uint32_t ns, uint32_t n
     return nullptr;
 }
 
-// The kernel of a pipelined one's geometry and ring depth for rows at any 2-byte alignment.
-const Variant *find_unaligned(const Variant &base, uint32_t nstage) {
+// The `_unaligned` kernel of a geometry, for slices at any 2-byte alignment.
+const Variant *find_unaligned(uint32_t d, uint32_t nq, uint32_t ns, uint32_t nstage, bool causal, bool bf16) {
     for (const auto &v : kVariants)
-        if (v.family == Family::kPipe && !v.aligned && v.d == base.d && v.nq == base.nq && v.ns == base.ns &&
-            v.nstage == nstage && v.causal == base.causal && v.bf16 == base.bf16)
+        if (v.family == Family::kPipe && !v.aligned && v.d == d && v.nq == nq && v.ns == ns && v.nstage == nstage &&
+            v.causal == causal && v.bf16 == bf16)
             return &v;
     return nullptr;
 }
@@ -412,14 +410,24 @@ const Variant *choose_pipe_layout(const nc_flash_options &o) {
     return best;
 }
 
-// Slices at odd elements: the pipelined choice in its `_unaligned` form (two stages where that has
-// three). Measured on MI355X with the reference's odd slice pads (17, 19, 23, 29), generic kernels ->
-// these: BH=8 S=1024 d=64 causal 19.3 -> 7.5 us, BH=16 S=1500 d=64 43.6 -> 20.3, BH=32 S=4096 d=64
-// 267 -> 152, BH=128 S=1000 d=32 causal 30.8 -> 21.4, BH=64 S=2048 d=16 88 -> 51, BH=3 S=49 d=16 causal
-// 3.21 -> 3.20 us; 16-byte aligned slices of the same shapes run 5.6, 18.0, 154, 19.6, 51 and 2.5 us.
+// Slices off 16-byte alignment. A row's exactness grows with its key splits (flash_fwd.hip, kGap), so
+// the geometry has at least as many as the generic kernel these layouts would have otherwise: eight
+// where that has eight, else two or four. Two (64 rows, four waves: three workgroups per CU) where the
+// grid fills the chip with them and four would spend their 128-key blocks on padding, or many times
+// over; else four. One ring stage instead of two as for aligned slices. Measured on MI355X, odd slice
+// pads (17, 19, 23, 29), us, generic / 2 splits / 4 / 8: BH=192 S=333 d=64 causal 27.3 / 14.4 / 18.5 / 20.9,
+// BH=64 S=4096 d=64 causal 281 / 205 / 212 / 272, BH=32 S=4096 d=64 262 / 201 / 196 / 240, BH=16 S=4096 d=64
+// causal 94.9 / 56.2 / 54.9 / 66.4, BH=128 S=1000 d=32 causal 32.3 / 21.8 / 26.0 / 35.9, BH=200 S=150 d=16
+// 6.4 / 6.1 / 7.2 / 6.2, BH=64 S=2048 d=16 93 / 60.9 / 57.9 / 63.4; eight in the generic kernel too: BH=8
+// S=1024 d=64 causal 19.0 -> 7.5, BH=24 S=1000 d=32 causal 15.7 -> 9.5, BH=3 S=49 d=16 causal 3.44 -> 3.12.
 const Variant *choose_unaligned(const nc_flash_options &o) {
-    const Variant *v = choose_pipe(o);
-    return v ? find_unaligned(*v, v->nq == 1 ? v->nstage : 2) : nullptr;
+    const uint32_t d = (uint32_t)o.head_dim;
+    const bool causal = o.causal != 0, bf = o.element_type == NC_ELEMENT_BF16;
+    const uint64_t S = o.seq_len, w64 = (S + 63) / 64 * o.batch_heads;
+    const Variant *g = choose_generic(o, false);
+    if (g && g->ns == 8) return find_unaligned(d, 1, 8, S <= (d == 64 && !causal ? 512u : 768u) ? 1 : 2, causal, bf);
+    const bool two = S <= 256 || (w64 >= 1024 && S <= 1536) || w64 >= 3072;
+    return find_unaligned(d, 2, two ? 2 : 4, 2, causal, bf);
 }
 
 uintptr_t address(const void *p) { return reinterpret_cast<uintptr_t>(p); }
@@ -446,18 +454,15 @@ int select_impl(const nc_flash_options *opts, uintptr_t low, uintptr_t olow, nc_
                             o.o_stride % 4 == 0 && rows[0] % 8 == 0 && rows[1] % 8 == 0 && rows[2] % 8 == 0 &&
                             rows[3] % 4 == 0;
     const bool aligned = ((low | olow) & 15u) == 0 && strides_ok;
-    // The pipelined kernels' 16-byte loads need every Q/K/V row to start at a dword (measured: the rate
-    // of aligned ones, buffer->LDS 147 GB/s per CU either way), their stores an O row at a float; their `_unaligned` forms take Q, K and V at any element, with one even row stride for K and V.
-    const bool o_floats = (olow & 3u) == 0;
-    const bool dwords = o_floats && (low & 3u) == 0 &&
-                        ((o.q_stride | o.k_stride | o.v_stride | rows[0] | rows[1] | rows[2]) & 1u) == 0;
-    const bool elements = o_floats && (low & 1u) == 0 && (rows[1] & 1u) == 0 && rows[1] == rows[2];
+    // The `_unaligned` pipelined kernels take Q, K and V at any element, with one even row stride for K
+    // and V, and store O at any float.
+    const bool elements = (olow & 3u) == 0 && (low & 1u) == 0 && (rows[1] & 1u) == 0 && rows[1] == rows[2];
     // The pipelined kernels address each Q/K/V slice with 32-bit buffer offsets, including up to
     // one block (<= 256 rows) past seq_len.
     uint64_t max_row = rows[0] > rows[1] ? rows[0] : rows[1];
     max_row = max_row > rows[2] ? max_row : rows[2];
     const bool offsets_fit = max_row < (1ull << 30) && (o.seq_len + 512) * max_row * 2 < (1ull << 31);
-    const Variant *v = offsets_fit && dwords     ? choose_pipe(o)
+    const Variant *v = offsets_fit && aligned    ? choose_pipe(o)
                        : offsets_fit && elements ? choose_unaligned(o)
                                                  : choose_generic(o, aligned);
     // A grid past the dispatch packet's work-items (below) on more threads than the generic kernel's.
@@ -471,8 +476,6 @@ int select_impl(const nc_flash_options *opts, uintptr_t low, uintptr_t olow, nc_
     // BH=1 S=8192 23.4 -> 18.6 us, BH=2 S=4096 13.4 -> 12.3 us, but c3 (32 query blocks) 5.9 -> 7.5 us
     // and grids beyond 256 workgroups slower too.
     const uint64_t nqb32 = (o.seq_len + 31) / 32;
-    // Only on 16-byte aligned slices: its scratch must not be shared by launches that overlap, and the
-    // other layouts' kernels have never needed any.
     if (v->family == Family::kPipe && aligned && v->causal && v->nq == 1 && v->d == 64 && nqb32 >= 96 &&
         nqb32 * o.batch_heads <= 256 && xsplit_pairs(o.batch_heads, o.seq_len) <= NC_XS_MAX_PAIRS) {
         const Variant *x = find_xsplit(v->d, v->bf16);

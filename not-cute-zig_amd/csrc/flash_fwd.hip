@@ -452,7 +452,7 @@ __device__ __forceinline__ void flash_fwd_body(const nc_flash_kernel_args &a) {
 
 
 // ---------------------------------------------------------------------------------------------
-// Pipelined variant (dword-aligned rows, in its UN form any slices; below 2 GiB): K and V stream through an
+// Pipelined variant (16-byte aligned rows, in its UN form any slices; below 2 GiB): K and V stream through an
 // NSTAGE-deep LDS ring by direct buffer->LDS loads (buffer_load_dwordx4 ... lds), so no VGPRs or
 // ds_write instructions are spent on staging and NSTAGE-1 blocks are always in flight. The buffer
 // descriptors cover exactly each slice's active rows, so key rows past seq_len read as zero
@@ -749,7 +749,8 @@ constexpr int pipe_lds_bytes() {
 // Odd slice pads, us: element-wise generic kernels / staging through registers with a funnel shift
 // per chunk (148-176 VGPRs, half the workgroups per CU) / shifting each chunk in place in LDS / this:
 // BH=8 S=1024 d=64 causal 19.3 / 8.7 / 11.1 / 7.5, BH=32 S=4096 d=64 267 / 209 / 181 / 152, BH=16 S=1500
-// d=64 35.4 / 31.0 / 27.9 / 20.3 (16-byte aligned slices: 5.6, 154, 18.0).
+// d=64 35.4 / 31.0 / 27.9 / 20.3 (16-byte aligned slices: 5.6, 154, 18.0), all four with a lazy running
+// max; with the exact one (kGap below) the kernels that are kept take 7.5, 196 and 21.2.
 template <int D, int NQ, int NS, bool CAUSAL, int NSTAGE, int SUB, bool BF, bool XS = false, bool UN = false,
           typename SlotFn>
 __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &a, char *smem, SlotFn &&slot_of) {
@@ -1071,12 +1072,20 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // to a weight that overflowed or is NaN, so such a tile's sums are not used: its redo adds each
     // lane's own weights by v_dot2c. The private-staging kernels of d = 32 and 64, whose few waves wait
     // on the tile's serial chain (S^T, weights, sum, PV), lose by the longer one (c3 5.59 -> 5.87 us), and
-    // the odd-slice q8s1 kernel has no registers for it: v_dot2c there.
+    // the `_unaligned` kernels have no check that would keep a NaN in its row: v_dot2c there.
     // Measured against v_dot2c (with the first tile's max and one check per tile below): BH=32 S=4096
     // d=64 146.9 -> 139.8 us, BH=64 S=4096 d=64 causal 156.6 -> 146.2, BH=128 S=512 d=64 causal 11.85 ->
     // 10.97, BH=4 S=8192 d=64 causal 54.9 -> 50.9, BH=32 S=4096 d=32 104.8 -> 101.8, BH=64 S=2048 d=16
     // 48.8 -> 45.7.
-    constexpr bool MSUM = D == 16 || (!PRIV && !(UN && NQ == 8));
+    constexpr bool MSUM = !UN && (D == 16 || !PRIV);
+    // UN moves the running max ahead of a tile's weights whenever the tile's max is above it by more than
+    // kGap (log2 units), as the generic kernels these layouts had did at every tile (kGap 0). The
+    // largest weight of a row is then exactly 1, and unrounded; with the lazy max of the aligned kernels
+    // peaked rows (logits of sigma 3) were off by up to 3.6e-5 from float64 where the generic kernel's
+    // are by 1.9e-5. Each key split has such a weight, so kernels with more splits may wait for a larger
+    // step, which saves rescales, and stay below the generic kernels' error: rms at BH=16 S=4096 d=64
+    // causal 2.9e-5 for the generic kernel and q2s2, 2.3e-5 q2s4, 1.7e-5 q1s8.
+    constexpr float kGap = NS >= 8 ? 1.f : NS == 4 ? 0.5f : 0.f;
     u32x4 ones = {0u, 0u, 0u, 0u};
     if (MSUM && ((lane >> 2) & 1) == ((lane >> 4) & 1)) {
         const uint32_t one2 = BF ? 0x3f803f80u : 0x3c003c00u;
@@ -1090,7 +1099,8 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     float mrow = neg_inf();  // running max of sc * score (log2 domain); -inf: none yet (MSUM: -neg_m)
     // What the weights are formed with: -mrow; while mrow is -inf, 0, or with MSUM +inf, so that the
     // first tile a row sees overflows and takes its max without a test of its own.
-    float neg_m = MSUM ? __builtin_inff() : 0.f;
+    // UN: a huge finite value, which any visible score exceeds and a masked one (-inf) does not.
+    float neg_m = MSUM ? __builtin_inff() : UN ? 3.4028235e38f : 0.f;
     float l = 0.f;  // row sum: this lane's keys, with MSUM all of the wave's
     floatx16 o[C::MT];
 #pragma unroll
@@ -1188,24 +1198,24 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
             }
             return ls;
         };
-        // Move the running max to the tile max (rows whose max does not grow keep it) and rescale.
-        auto to_tile_max = [&]() {
+        // Largest score of the lane's 16. (Folding -inf in first lets the compiler fuse the tree into
+        // v_max3 without extra canonicalising maxes.)
+        auto lane_max = [&]() {
             const floatx16 &x = acc;
-            float tmax;
+            const float m0 = fmaxf(fmaxf(x[0], x[1]), x[2]), m1 = fmaxf(fmaxf(x[3], x[4]), x[5]);
+            const float m2 = fmaxf(fmaxf(x[6], x[7]), x[8]), m3 = fmaxf(fmaxf(x[9], x[10]), x[11]);
+            const float m4 = fmaxf(fmaxf(x[12], x[13]), x[14]);
+            return fmaxf(neg_inf(), fmaxf(fmaxf(fmaxf(m0, m1), m2), fmaxf(fmaxf(m3, m4), x[15])));
+        };
+        // Move the running max to the tile max (rows whose max does not grow keep it) and rescale.
+        auto to_tile_max = [&](float tmax) {
             if constexpr (MSUM) {
                 tmax = neg_inf();
                 asm volatile("" : "+v"(tmax));  // or the compiler forms it beside every tile's weights
 #pragma unroll
-                for (int r = 0; r < 16; r += 2) tmax = fmaxf(fmaxf(tmax, x[r]), x[r + 1]);
-                mrow = -neg_m;
-            } else {
-                const float m0 = fmaxf(fmaxf(x[0], x[1]), x[2]), m1 = fmaxf(fmaxf(x[3], x[4]), x[5]);
-                const float m2 = fmaxf(fmaxf(x[6], x[7]), x[8]), m3 = fmaxf(fmaxf(x[9], x[10]), x[11]);
-                const float m4 = fmaxf(fmaxf(x[12], x[13]), x[14]);
-                // (folding -inf in first lets the compiler fuse the tree into v_max3 without extra
-                // canonicalising maxes)
-                tmax = fmaxf(neg_inf(), fmaxf(fmaxf(fmaxf(m0, m1), m2), fmaxf(fmaxf(m3, m4), x[15])));
+                for (int r = 0; r < 16; r += 2) tmax = fmaxf(fmaxf(tmax, acc[r]), acc[r + 1]);
             }
+            if constexpr (MSUM || UN) mrow = -neg_m;
             const float m_new = fmaxf(mrow, pair_max(tmax) * sc);
             const float alpha = __builtin_amdgcn_exp2f(mrow - (m_new == neg_inf() ? 0.f : m_new));
             l *= alpha;
@@ -1215,7 +1225,11 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
             neg_m = (mrow == neg_inf()) ? 0.f : -mrow;
         };
         float ls = 0.f;
-        if constexpr (MSUM) {
+        if constexpr (UN) {
+            const float tmax = lane_max();
+            if (__builtin_amdgcn_ballot_w64(__builtin_fmaf(tmax, sc, neg_m) > kGap)) to_tile_max(tmax);
+            ls = weights(IC<0>{});
+        } else if constexpr (MSUM) {
             // (the first tile's max is taken at once, every other one's when its sums show the need)
             bool redo = first;
             if (!first) {
@@ -1223,17 +1237,17 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
                 redo = __builtin_amdgcn_ballot_w64(!(ls < weight_sum_limit<BF>())) != 0;
             }
             if (redo) {
-                to_tile_max();
+                to_tile_max(0.f);
                 ls = pair_sum(weights(IC<0>{}));
                 if (mrow == neg_inf()) neg_m = __builtin_inff();  // a row that has seen no key yet
             }
         } else if (__builtin_amdgcn_ballot_w64(mrow == neg_inf())) {
-            to_tile_max();  // some row has no max yet: take it first
+            to_tile_max(lane_max());  // some row has no max yet: take it first
             ls = weights(IC<0>{});
         } else {
             ls = weights(IC<0>{});
             if (__builtin_amdgcn_ballot_w64(!(ls < weight_sum_limit<BF>()))) {
-                to_tile_max();  // a weight overflowed (f16) or grew too large (bf16): redo the tile
+                to_tile_max(lane_max());  // a weight overflowed (f16) or grew too large (bf16): redo the tile
                 ls = weights(IC<0>{});
             }
         }
@@ -1403,7 +1417,7 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     };
     float2v *mlb = reinterpret_cast<float2v *>(smem + C::ML_OFF);  // [BM queries][NS splits]
     const float lt = MSUM ? l : pair_sum(l);
-    if constexpr (MSUM) mrow = -neg_m;
+    if constexpr (MSUM || UN) mrow = -neg_m;
     if constexpr (PRIV && NS > 1) {
         // Epilogue, private staging: once a wave is past its loop, the K and V slices of ring
         // stage 0 that only it ever loaded are free, so it writes its unscaled O^T partial there
@@ -2318,28 +2332,26 @@ NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_causal, 64, 1, 8, true, 2, 1)
     void NAME##_bf16(nc_flash_kernel_args a) {                                                          \
         flash_fwd_pipe_kernel<D, NQ, NS, CAUSAL, NSTAGE, SUB, true, false, true>(a);                      \
     }
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q8s1p2t2_full_unaligned, 64, 8, 1, false, 2, 2, 4)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q8s1p2t2_causal_unaligned, 64, 8, 1, true, 2, 2, 4)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q4s1p2t2_full_unaligned, 64, 4, 1, false, 2, 2, 3)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q4s1p2t2_causal_unaligned, 64, 4, 1, true, 2, 2, 3)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_full_unaligned, 64, 2, 4, false, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_causal_unaligned, 64, 2, 4, true, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s2p2_full_unaligned, 64, 2, 2, false, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s2p2_causal_unaligned, 64, 2, 2, true, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_full_unaligned, 64, 1, 8, false, 2, 1, 2)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_causal_unaligned, 64, 1, 8, true, 2, 1, 2)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p1_full_unaligned, 64, 1, 8, false, 1, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p1_causal_unaligned, 64, 1, 8, true, 1, 1, 4)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q4s1p2_full_unaligned, 32, 4, 1, false, 2, 1, 5)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q4s1p2_causal_unaligned, 32, 4, 1, true, 2, 1, 5)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s4p2_full_unaligned, 32, 2, 4, false, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s4p2_causal_unaligned, 32, 2, 4, true, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s2p2_full_unaligned, 32, 2, 2, false, 2, 1, 5)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s2p2_causal_unaligned, 32, 2, 2, true, 2, 1, 5)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p2_full_unaligned, 32, 1, 8, false, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p2_causal_unaligned, 32, 1, 8, true, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p1_full_unaligned, 32, 1, 8, false, 1, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p1_causal_unaligned, 32, 1, 8, true, 1, 1, 4)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q4s1p2t2_full_unaligned, 16, 4, 1, false, 2, 2, 5)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q4s1p2t2_causal_unaligned, 16, 4, 1, true, 2, 2, 5)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s4p2_full_unaligned, 16, 2, 4, false, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s4p2_causal_unaligned, 16, 2, 4, true, 2, 1, 4)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s2p2_full_unaligned, 16, 2, 2, false, 2, 1, 5)
+NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s2p2_causal_unaligned, 16, 2, 2, true, 2, 1, 5)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q1s8p2_full_unaligned, 16, 1, 8, false, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q1s8p2_causal_unaligned, 16, 1, 8, true, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q1s8p1_full_unaligned, 16, 1, 8, false, 1, 1, 4)

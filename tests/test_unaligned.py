@@ -1,6 +1,5 @@
-"""Dispatch of slices that are not 16-byte aligned (no GPU): the pipelined kernels take every layout
-whose Q/K/V rows start at dwords, their `_unaligned` forms any 2-byte alignment with one even row
-stride for K and V, and the generic kernels the rest."""
+"""Dispatch of slices that are not 16-byte aligned (no GPU): the `_unaligned` pipelined kernels take
+every layout at elements with one even row stride for K and V, the generic kernels the rest."""
 
 import itertools
 
@@ -32,17 +31,17 @@ def test_route_follows_the_layout(bh, s, d, causal):
     for offs in itertools.product((0, 1, 2, 4), repeat=3):  # elements past 16-byte alignment of Q, K, V
         ptr = dict(zip("qkv", (BASE + 2 * x for x in offs)))
         family, sel = route(bh, s, d, causal, **ptr)
-        assert family == ("unaligned" if 1 in offs else "pipe"), offs
+        assert family == ("unaligned" if any(offs) else "pipe"), offs
         assert sel.aligned == (1 if not any(offs) else 0)
     for pads in itertools.product((0, 3, 6), repeat=3):
         family, sel = route(bh, s, d, causal, pads=pads + (5,))
-        assert family == ("unaligned" if 3 in pads else "pipe"), pads
+        assert family == "unaligned", pads  # (the float padding of O alone is enough)
         assert sel.aligned == 0
     # O: any float; an address between floats, and odd, differing or odd-element K/V rows: generic
-    assert route(bh, s, d, causal, o=BASE + 4)[0] == "pipe"
+    assert route(bh, s, d, causal, o=BASE + 4)[0] == "unaligned"
     assert route(bh, s, d, causal, o=BASE + 2)[0] == "generic"
     assert route(bh, s, d, causal, q=BASE + 1)[0] == "generic"
-    assert route(bh, s, d, causal, rows=(d + 2, d + 2, d + 4, d + 1))[0] == "pipe"
+    assert route(bh, s, d, causal, rows=(d + 2, d + 2, d + 4, d + 1))[0] == "generic"
     assert route(bh, s, d, causal, rows=(d + 1, d + 2, d + 2, 0))[0] == "unaligned"
     assert route(bh, s, d, causal, k=BASE + 2, rows=(0, d + 2, d + 4, 0))[0] == "generic"
     assert route(bh, s, d, causal, rows=(0, d + 1, d + 1, 0))[0] == "generic"
@@ -52,15 +51,18 @@ def test_route_follows_the_layout(bh, s, d, causal):
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_unaligned_selection_is_launchable(bh, s, d, dtype):
     for causal in (False, True):
-        _, al = route(bh, s, d, causal, dtype=dtype)
+        # an odd K/V row stride: the generic kernel
+        _, gen = route(bh, s, d, causal, rows=(0, d + 1, d + 1, 0), dtype=dtype)
         _, un = route(bh, s, d, causal, k=BASE + 2, dtype=dtype)
         assert un.name.decode().endswith("_unaligned_bf16" if dtype == "bf16" else "_unaligned")
-        assert un.block_m == al.block_m and un.threads == al.threads and un.scratch_bytes == 0
+        # (threads per row: 2 per key split) no fewer splits than the generic kernel, since a row's
+        # exactness grows with them
+        assert un.threads // un.block_m >= gen.threads // gen.block_m and un.scratch_bytes == 0
         assert un.grid[0] == -(-s // un.block_m) * bh and un.grid[1] == un.grid[2] == 1
 
 
 def test_no_new_scratch_and_no_new_refusals():
-    """The pair split's scratch stays with 16-byte aligned slices, and a grid that only the generic
+    """The pair split's scratch stays with 16-byte aligned slices; a grid that only the generic
     kernels' workgroups fit keeps them."""
     assert route(1, 4096, 64, True)[1].scratch_bytes > 0
     for ptr in (BASE + 4, BASE + 2):
