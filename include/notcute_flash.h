@@ -259,7 +259,7 @@ typedef struct nc_flash_kernel_selection {
  * at that size, where no packed-slice 3-D grid applies). */
 int nc_flash_select_kernel(const nc_flash_options *opts, nc_flash_kernel_selection *out);
 
-/* Same, for the actual buffers: picks the element-wise variant when a pointer or stride breaks
+/* Same, for the actual buffers: picks an `_unaligned` variant when a pointer or stride breaks
  * 16-byte alignment (the reference's smoke cases use odd slice pads, src/main.zig:190-193). */
 int nc_flash_select_kernel_for(const nc_flash_options *opts, const void *q, const void *k,
                                const void *v, const void *o, nc_flash_kernel_selection *out);
