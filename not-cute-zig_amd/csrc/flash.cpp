@@ -82,8 +82,7 @@ struct Variant {
 #define PIPEU(D, NQ, NS, P, C, T, BF) {"nc_flash_fwd_d" #D "_q" #NQ "s" #NS "p" #P "_" C "_unaligned" T, \
                                        D, NQ, NS, P, 1, C[0] == 'c', false, Family::kPipe, BF}
 #define PIPEU2(D, NQ, NS, P, T, BF) PIPEU(D, NQ, NS, P, "full", T, BF), PIPEU(D, NQ, NS, P, "causal", T, BF)
-#define PIPEU8(D, T, BF) PIPEU2(D, 2, 4, 2, T, BF), PIPEU2(D, 2, 2, 2, T, BF), PIPEU2(D, 1, 8, 2, T, BF), \
-    PIPEU2(D, 1, 8, 1, T, BF)
+#define PIPEU6(D, T, BF) PIPEU2(D, 2, 2, 2, T, BF), PIPEU2(D, 1, 8, 2, T, BF), PIPEU2(D, 1, 8, 1, T, BF)
 #define GEN(D, C, A, SUF, T, BF) {"nc_flash_fwd_d" #D "_m64_" C SUF T, D, 2, 2, 1, 1, C[0] == 'c', A, \
                                   Family::kGeneric, BF}
 // The generic body in other geometries (32 rows x 8 key splits; 128 rows x 2 key splits).
@@ -109,7 +108,7 @@ struct Variant {
     PIPE(64, 1, 8, 1, "full", T, BF), PIPE(64, 1, 8, 1, "causal", T, BF), PIPE(32, 1, 8, 1, "full", T, BF),   \
     PIPE(32, 1, 8, 1, "causal", T, BF), PIPE(16, 1, 8, 1, "full", T, BF), PIPE(16, 1, 8, 1, "causal", T, BF), \
     PIPED4(64, T, BF), PIPED4(32, T, BF), PIPED4(16, T, BF),                                                  \
-    PIPEU8(64, T, BF), PIPEU8(32, T, BF), PIPEU8(16, T, BF)
+    PIPEU6(64, T, BF), PIPEU6(32, T, BF), PIPEU6(16, T, BF)
 
 const Variant kVariants[] = {VARIANTS("", false), VARIANTS("_bf16", true)};
 #undef VARIANTS
@@ -120,7 +119,7 @@ const Variant kVariants[] = {VARIANTS("", false), VARIANTS("_bf16", true)};
 #undef PIPED4
 #undef PIPEU
 #undef PIPEU2
-#undef PIPEU8
+#undef PIPEU6
 #undef GEN
 #undef GENG
 #undef GENG2
@@ -410,24 +409,20 @@ const Variant *choose_pipe_layout(const nc_flash_options &o) {
     return best;
 }
 
-// Slices off 16-byte alignment. A row's exactness grows with its key splits (flash_fwd.hip, kGap), so
-// the geometry has at least as many as the generic kernel these layouts would have otherwise: eight
-// where that has eight, else two or four. Two (64 rows, four waves: three workgroups per CU) where the
-// grid fills the chip with them and four would spend their 128-key blocks on padding, or many times
-// over; else four. One ring stage instead of two as for aligned slices. Measured on MI355X, odd slice
-// pads (17, 19, 23, 29), us, generic / 2 splits / 4 / 8: BH=192 S=333 d=64 causal 27.3 / 14.4 / 18.5 / 20.9,
-// BH=64 S=4096 d=64 causal 281 / 205 / 212 / 272, BH=32 S=4096 d=64 262 / 201 / 196 / 240, BH=16 S=4096 d=64
-// causal 94.9 / 56.2 / 54.9 / 66.4, BH=128 S=1000 d=32 causal 32.3 / 21.8 / 26.0 / 35.9, BH=200 S=150 d=16
-// 6.4 / 6.1 / 7.2 / 6.2, BH=64 S=2048 d=16 93 / 60.9 / 57.9 / 63.4; eight in the generic kernel too: BH=8
-// S=1024 d=64 causal 19.0 -> 7.5, BH=24 S=1000 d=32 causal 15.7 -> 9.5, BH=3 S=49 d=16 causal 3.44 -> 3.12.
+// Slices off 16-byte alignment: as many key splits as the generic kernel these layouts would have
+// otherwise, eight (32 rows) or two (64 rows, four waves: three workgroups per CU and more), so that a
+// row's weights are rounded at the same running maxima and the output is the same but for the rounding
+// of f32 sums (flash_fwd.hip, UN). Four splits are up to 20 % faster on mid-size grids (BH=16 S=1500 d=64
+// 23.2 -> 20.4 us), but round each weight elsewhere. Measured on MI355X, odd slice pads (17, 19, 23, 29),
+// us, generic -> here: BH=192 S=333 d=64 causal bf16 27.1 -> 15.7, BH=64 S=4096 d=64 causal 266 -> 206,
+// BH=32 S=4096 d=64 275 -> 207, BH=64 S=2048 d=16 88.0 -> 60.6, BH=32 S=4096 d=32 186 -> 134; eight splits:
+// BH=8 S=250 d=32 causal 5.47 -> 4.38, BH=4 S=1979 d=64 31.2 -> 12.3, BH=1 S=32 d=16 3.61 -> 3.13.
 const Variant *choose_unaligned(const nc_flash_options &o) {
     const uint32_t d = (uint32_t)o.head_dim;
     const bool causal = o.causal != 0, bf = o.element_type == NC_ELEMENT_BF16;
-    const uint64_t S = o.seq_len, w64 = (S + 63) / 64 * o.batch_heads;
     const Variant *g = choose_generic(o, false);
-    if (g && g->ns == 8) return find_unaligned(d, 1, 8, S <= (d == 64 && !causal ? 512u : 768u) ? 1 : 2, causal, bf);
-    const bool two = S <= 256 || (w64 >= 1024 && S <= 1536) || w64 >= 3072;
-    return find_unaligned(d, 2, two ? 2 : 4, 2, causal, bf);
+    if (!g || g->ns != 8) return find_unaligned(d, 2, 2, 2, causal, bf);
+    return find_unaligned(d, 1, 8, o.seq_len <= (d == 64 && !causal ? 512u : 768u) ? 1 : 2, causal, bf);
 }
 
 uintptr_t address(const void *p) { return reinterpret_cast<uintptr_t>(p); }
@@ -465,9 +460,6 @@ int select_impl(const nc_flash_options *opts, uintptr_t low, uintptr_t olow, nc_
     const Variant *v = offsets_fit && aligned    ? choose_pipe(o)
                        : offsets_fit && elements ? choose_unaligned(o)
                                                  : choose_generic(o, aligned);
-    // A grid past the dispatch packet's work-items (below) on more threads than the generic kernel's.
-    if (v && !aligned && (o.seq_len + v->bm() - 1) / v->bm() > 0xffffffffull / v->threads() / o.batch_heads)
-        v = choose_generic(o, aligned);
     if (!v) return NC_ERROR_NOT_FOUND;
     // Long causal sequences over few heads on the private-staging kernel: pair the light and heavy
     // query blocks so that every workgroup takes about half the heaviest block's keys. It pays once

@@ -750,7 +750,7 @@ constexpr int pipe_lds_bytes() {
 // per chunk (148-176 VGPRs, half the workgroups per CU) / shifting each chunk in place in LDS / this:
 // BH=8 S=1024 d=64 causal 19.3 / 8.7 / 11.1 / 7.5, BH=32 S=4096 d=64 267 / 209 / 181 / 152, BH=16 S=1500
 // d=64 35.4 / 31.0 / 27.9 / 20.3 (16-byte aligned slices: 5.6, 154, 18.0), all four with a lazy running
-// max; with the exact one (kGap below) the kernels that are kept take 7.5, 196 and 21.2.
+// max; with the exact one (below) the kernels that are kept take 7.5, 207 and 23.2.
 template <int D, int NQ, int NS, bool CAUSAL, int NSTAGE, int SUB, bool BF, bool XS = false, bool UN = false,
           typename SlotFn>
 __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &a, char *smem, SlotFn &&slot_of) {
@@ -1078,14 +1078,12 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // 10.97, BH=4 S=8192 d=64 causal 54.9 -> 50.9, BH=32 S=4096 d=32 104.8 -> 101.8, BH=64 S=2048 d=16
     // 48.8 -> 45.7.
     constexpr bool MSUM = !UN && (D == 16 || !PRIV);
-    // UN moves the running max ahead of a tile's weights whenever the tile's max is above it by more than
-    // kGap (log2 units), as the generic kernels these layouts had did at every tile (kGap 0). The
-    // largest weight of a row is then exactly 1, and unrounded; with the lazy max of the aligned kernels
-    // peaked rows (logits of sigma 3) were off by up to 3.6e-5 from float64 where the generic kernel's
-    // are by 1.9e-5. Each key split has such a weight, so kernels with more splits may wait for a larger
-    // step, which saves rescales, and stay below the generic kernels' error: rms at BH=16 S=4096 d=64
-    // causal 2.9e-5 for the generic kernel and q2s2, 2.3e-5 q2s4, 1.7e-5 q1s8.
-    constexpr float kGap = NS >= 8 ? 1.f : NS == 4 ? 0.5f : 0.f;
+    // UN moves the running max to a tile's max ahead of its weights, as the generic kernels that these
+    // layouts have otherwise do, and is dispatched with their number of key splits: a row's weights are
+    // then rounded at the same maxima, so that the two differ by the rounding of their f32 sums alone.
+    // (The lazy max of the aligned kernels doubled the error of peaked rows: logits of sigma 3, 1.9e-5 ->
+    // 3.6e-5 at most. Waiting for a step of 1 with eight splits raised its rms by 1 %.) Against the generic
+    // kernels, 2-norm, BH=16 S=1500 d=64: 7.8e-6 (f16), where both are 1.8e-4 off float64.
     u32x4 ones = {0u, 0u, 0u, 0u};
     if (MSUM && ((lane >> 2) & 1) == ((lane >> 4) & 1)) {
         const uint32_t one2 = BF ? 0x3f803f80u : 0x3c003c00u;
@@ -1227,7 +1225,7 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
         float ls = 0.f;
         if constexpr (UN) {
             const float tmax = lane_max();
-            if (__builtin_amdgcn_ballot_w64(__builtin_fmaf(tmax, sc, neg_m) > kGap)) to_tile_max(tmax);
+            if (__builtin_amdgcn_ballot_w64(__builtin_fmaf(tmax, sc, neg_m) > 0.f)) to_tile_max(tmax);
             ls = weights(IC<0>{});
         } else if constexpr (MSUM) {
             // (the first tile's max is taken at once, every other one's when its sums show the need)
@@ -2334,24 +2332,18 @@ NC_FLASH_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_causal, 64, 1, 8, true, 2, 1)
     void NAME##_bf16(nc_flash_kernel_args a) {                                                          \
         flash_fwd_pipe_kernel<D, NQ, NS, CAUSAL, NSTAGE, SUB, true, false, true>(a);                      \
     }
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_full_unaligned, 64, 2, 4, false, 2, 1, 4)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s4p2_causal_unaligned, 64, 2, 4, true, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s2p2_full_unaligned, 64, 2, 2, false, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q2s2p2_causal_unaligned, 64, 2, 2, true, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_full_unaligned, 64, 1, 8, false, 2, 1, 2)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p2_causal_unaligned, 64, 1, 8, true, 2, 1, 2)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p1_full_unaligned, 64, 1, 8, false, 1, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d64_q1s8p1_causal_unaligned, 64, 1, 8, true, 1, 1, 4)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s4p2_full_unaligned, 32, 2, 4, false, 2, 1, 4)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s4p2_causal_unaligned, 32, 2, 4, true, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s2p2_full_unaligned, 32, 2, 2, false, 2, 1, 5)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q2s2p2_causal_unaligned, 32, 2, 2, true, 2, 1, 5)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p2_full_unaligned, 32, 1, 8, false, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p2_causal_unaligned, 32, 1, 8, true, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p1_full_unaligned, 32, 1, 8, false, 1, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d32_q1s8p1_causal_unaligned, 32, 1, 8, true, 1, 1, 4)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s4p2_full_unaligned, 16, 2, 4, false, 2, 1, 4)
-NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s4p2_causal_unaligned, 16, 2, 4, true, 2, 1, 4)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s2p2_full_unaligned, 16, 2, 2, false, 2, 1, 5)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q2s2p2_causal_unaligned, 16, 2, 2, true, 2, 1, 5)
 NC_FLASH_UNALIGNED_PIPE_KERNEL(nc_flash_fwd_d16_q1s8p2_full_unaligned, 16, 1, 8, false, 2, 1, 4)

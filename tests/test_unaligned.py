@@ -72,3 +72,15 @@ def test_no_new_scratch_and_no_new_refusals():
             family, sel = route((1 << 23) - 1, 1, d, False, q=ptr)
             assert sel.grid[0] * sel.threads <= 0xFFFFFFFF
     assert route((1 << 24) - 1, 1, 32, False, q=BASE + 2)[1].threads == 256
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("causal", [False, True])
+def test_key_splits_are_the_generic_kernels(d, causal):
+    """A weight is rounded at the running max of its key split, so a call's output stays what the generic
+    kernel gives it only with that kernel's number of splits."""
+    for bh in (1, 3, 8, 16, 24, 64, 100, 192, 500):
+        for s in (1, 32, 33, 129, 250, 333, 700, 1500, 2048, 4096, 8192):
+            gen = route(bh, s, d, causal, rows=(0, d + 1, d + 1, 0))[1]
+            for ptr in (BASE + 2, BASE + 4):
+                assert route(bh, s, d, causal, k=ptr)[1].kv_splits == gen.kv_splits, (bh, s)

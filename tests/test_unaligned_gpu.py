@@ -142,3 +142,43 @@ def test_peaked_rows_are_as_exact_as_the_generic_kernels(gpu, bh, s, d, causal, 
     print(f"[ok] {errs}", flush=True)
     assert errs["unaligned"][0] <= 1.25 * errs["generic"][0]
     assert errs["unaligned"][1] <= 1.05 * errs["generic"][1]
+
+
+@pytest.mark.parametrize("bh,s,d,causal", [(16, 1500, 64, False), (32, 700, 64, True), (8, 250, 32, True),
+                                           (96, 520, 32, False), (64, 1100, 16, True), (4, 1979, 64, False)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_output_is_the_generic_kernels(gpu, bh, s, d, causal, dtype):
+    """Both round a weight at the same running max, so they differ only where an exponent's f32 rounding
+    (of |scores| up to 8: four units of 2^-21) takes a weight across the middle between two neighbours,
+    2^-11 or more apart (f16): at most a share 2 * 4 * 2^-21 * ln 2 / 2^-11 of the weights, by sqrt(12)
+    times the rms rounding error each. That is sqrt(12 * 0.0054) = 0.25 of the error against float64;
+    0.3 with the sums' own rounding. Weights rounded at other maxima differ by 0.8 of it and more."""
+    wl = Workload(f"same_{bh}_{s}_{d}", bh, s, d, causal, 1.0 / math.sqrt(d), (("normal", 0.0, 1.0),) * 3, seed=70,
+                  q_stride=s * d + 17, k_stride=s * d + 19, v_stride=s * d + 23, o_stride=s * d + 29, dtype=dtype)
+    tensors = wl.make_inputs()
+    rows = np.arange(0, s, max(1, s // 64))
+    idx = fc.active_index(wl, rows)
+    ref = fc.oracle(wl, *tensors, rows=rows)[idx].astype(np.float64)
+    odd = dataclasses.replace(wl, k_row=d + 1, v_row=d + 1, k_stride=0, v_stride=0)
+    o_init = np.full(wl.length("o"), fc.SENTINEL, np.float32)
+    bufs = [nc.DeviceBuffer.from_array(t) for t in (*tensors, o_init)]
+    out = {}
+    try:
+        ptr = [b.ptr for b in bufs]
+        for kind, opts in (("generic", odd.options()), ("unaligned", wl.options())):
+            sel = nc.select_kernel_for(opts, *ptr)
+            name = sel.name.decode()
+            print(f"[case] {wl.describe()} {dtype} {name}", flush=True)
+            assert ("_m64_" in name) == (kind == "generic")
+            bufs[3].upload(o_init)
+            args = nc.pack_args(wl.options(), sel, *ptr)
+            gpu.get_function(name).launch(tuple(sel.grid), (sel.threads,), nc.kernel_params(name, args))
+            nc.synchronize()
+            out[kind] = bufs[3].download(np.float32, wl.length("o"))[idx].astype(np.float64)
+    finally:
+        for b in bufs:
+            b.free()
+    err = np.linalg.norm(out["generic"] - ref)
+    diff = np.linalg.norm(out["unaligned"] - out["generic"])
+    print(f"[ok] difference {diff / np.linalg.norm(ref):.2e} error {err / np.linalg.norm(ref):.2e}", flush=True)
+    assert diff <= 0.3 * err
