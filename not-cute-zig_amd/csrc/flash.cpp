@@ -409,6 +409,30 @@ const Variant *choose_pipe_layout(const nc_flash_options &o) {
     return best;
 }
 
+// Whether the two-split `_unaligned` kernel (64 rows) is launched rather than the generic one `g`, dwords
+// saying that Q, K and V all start at whole dwords. The generic kernels load those as fast as aligned
+// rows, odd elements at a quarter of that rate. Times on MI355X as generic / here, us.
+//  - Against the 128-row generic kernel it reads K and V twice as often. That is free while the slices an
+//    XCD works through at a time (every 8th workgroup's) stay near its 4 MB L2: it pays below 12 MiB of K and
+//    V there, causal (half the reads) 32 MiB. BH=64 S=4000 (7.8 MiB) 491 / 383, BH=384 S=1021 (12.0)
+//    232 / 223, BH=120 S=4000 (14.6) 856 / 905, BH=199 S=4000 (194) 1469 / 1725; causal BH=300 S=1021 (18.7)
+//    122 / 107, BH=61 S=2048 (30.5) 80.0 / 73.4, BH=512 S=2048 (32.0) 625 / 633, BH=150 S=4000 (73) 594 / 679.
+//    Up to S = 384, few reads: odd slices BH=1023 S=256 (64) 58.8 / 56.8, dwords only in one block of 64
+//    rows (BH=5301 S=64 46.7 / 40.5); dwords in two 64-row blocks for one of 128 rows are a draw
+//    (BH=495 S=79 10.1 / 10.6, BH=664 S=105 16.4 / 12.7).
+//  - Against the 64-row ones, short sequences leave each wave one or two tiles: d = 16 and 32 up to S = 64
+//    (BH=820 S=18 d=16 4.5 / 5.2, BH=918 S=34 d=16 5.1 / 5.6), with dwords to 128 (BH=448 S=92 d=16 5.4 / 5.8),
+//    d=64 to 64 (BH=229 S=43 4.8 / 5.3).
+// Random shapes timed after these lines were drawn (BH 1-4000, S 4-8192, odd and dword slices): where an
+// `_unaligned` kernel is launched, 0.33-0.98 of the generic time, 0.72 in the geometric mean of 1004.
+bool two_splits_pay(const nc_flash_options &o, const Variant &g, bool dwords) {
+    const uint64_t S = o.seq_len, d = o.head_dim, bh = o.batch_heads;
+    if (g.bm() != 128) return S > (d == 64 ? (dwords ? 64u : 0u) : dwords ? 128u : 64u);
+    if (S <= (dwords ? 64u : 384u)) return true;
+    const uint64_t heads = bh / std::min<uint64_t>(bh & (~bh + 1), 8);  // of an XCD's workgroups
+    return !(dwords && S <= 128) && heads <= (((o.causal ? 32u : 12u) << 20) - 1) / (S * d * 4);
+}
+
 // Slices off 16-byte alignment: as many key splits as the generic kernel these layouts would have
 // otherwise, eight (32 rows) or two (64 rows, four waves: three workgroups per CU and more), so that a
 // row's weights are rounded at the same running maxima and the output is the same but for the rounding
@@ -417,11 +441,12 @@ const Variant *choose_pipe_layout(const nc_flash_options &o) {
 // us, generic -> here: BH=192 S=333 d=64 causal bf16 27.1 -> 15.7, BH=64 S=4096 d=64 causal 266 -> 206,
 // BH=32 S=4096 d=64 275 -> 207, BH=64 S=2048 d=16 88.0 -> 60.6, BH=32 S=4096 d=32 186 -> 134; eight splits:
 // BH=8 S=250 d=32 causal 5.47 -> 4.38, BH=4 S=1979 d=64 31.2 -> 12.3, BH=1 S=32 d=16 3.61 -> 3.13.
-const Variant *choose_unaligned(const nc_flash_options &o) {
+const Variant *choose_unaligned(const nc_flash_options &o, bool dwords) {
     const uint32_t d = (uint32_t)o.head_dim;
     const bool causal = o.causal != 0, bf = o.element_type == NC_ELEMENT_BF16;
     const Variant *g = choose_generic(o, false);
-    if (!g || g->ns != 8) return find_unaligned(d, 2, 2, 2, causal, bf);
+    if (!g) return nullptr;
+    if (g->ns != 8) return two_splits_pay(o, *g, dwords) ? find_unaligned(d, 2, 2, 2, causal, bf) : g;
     return find_unaligned(d, 1, 8, o.seq_len <= (d == 64 && !causal ? 512u : 768u) ? 1 : 2, causal, bf);
 }
 
@@ -452,13 +477,14 @@ int select_impl(const nc_flash_options *opts, uintptr_t low, uintptr_t olow, nc_
     // The `_unaligned` pipelined kernels take Q, K and V at any element, with one even row stride for K
     // and V, and store O at any float.
     const bool elements = (olow & 3u) == 0 && (low & 1u) == 0 && (rows[1] & 1u) == 0 && rows[1] == rows[2];
+    const bool dwords = ((low | 2 * (o.q_stride | rows[0] | o.k_stride | o.v_stride)) & 3u) == 0;
     // The pipelined kernels address each Q/K/V slice with 32-bit buffer offsets, including up to
     // one block (<= 256 rows) past seq_len.
     uint64_t max_row = rows[0] > rows[1] ? rows[0] : rows[1];
     max_row = max_row > rows[2] ? max_row : rows[2];
     const bool offsets_fit = max_row < (1ull << 30) && (o.seq_len + 512) * max_row * 2 < (1ull << 31);
     const Variant *v = offsets_fit && aligned    ? choose_pipe(o)
-                       : offsets_fit && elements ? choose_unaligned(o)
+                       : offsets_fit && elements ? choose_unaligned(o, dwords)
                                                  : choose_generic(o, aligned);
     if (!v) return NC_ERROR_NOT_FOUND;
     // Long causal sequences over few heads on the private-staging kernel: pair the light and heavy

@@ -84,3 +84,35 @@ def test_key_splits_are_the_generic_kernels(d, causal):
             gen = route(bh, s, d, causal, rows=(0, d + 1, d + 1, 0))[1]
             for ptr in (BASE + 2, BASE + 4):
                 assert route(bh, s, d, causal, k=ptr)[1].kv_splits == gen.kv_splits, (bh, s)
+
+
+@pytest.mark.parametrize("bh,s,d,causal,odd,dword", [
+    # K and V of an XCD's slices against its L2 (d = 64, the 128-row generic kernel otherwise)
+    (64, 4000, 64, False, "unaligned", "unaligned"), (199, 2048, 64, False, "generic", "generic"),
+    (199, 2048, 64, True, "generic", "generic"), (100, 4000, 64, False, "generic", "generic"),
+    (100, 4000, 64, True, "unaligned", "unaligned"), (333, 4000, 64, True, "generic", "generic"),
+    (4095, 512, 64, False, "generic", "generic"), (1023, 256, 64, False, "unaligned", "generic"),
+    (64, 8192, 64, True, "unaligned", "unaligned"), (5387, 368, 64, False, "unaligned", "generic"),
+    # few reads of K and V
+    (1000, 64, 64, False, "unaligned", "unaligned"), (495, 79, 64, True, "unaligned", "generic"),
+    # one or two tiles per wave (the 64-row generic kernel)
+    (229, 43, 64, False, "unaligned", "generic"), (820, 18, 16, False, "generic", "generic"),
+    (920, 65, 32, True, "unaligned", "generic"), (920, 129, 32, True, "unaligned", "unaligned"),
+    # eight key splits: always
+    (8, 20, 16, True, "unaligned", "unaligned"), (3, 8192, 64, True, "unaligned", "unaligned")])
+def test_generic_kernels_where_they_are_faster(bh, s, d, causal, odd, dword):
+    assert route(bh, s, d, causal, pads=(17, 19, 23, 29))[0] == odd
+    assert route(bh, s, d, causal, q=BASE + 2)[0] == odd
+    assert route(bh, s, d, causal, pads=(2, 6, 10, 3))[0] == dword
+    assert route(bh, s, d, causal, o=BASE + 4)[0] == dword
+
+
+def test_dispatch_holds_at_the_largest_sizes():
+    """No overflow in the rule: the largest counts still select a kernel or are refused for their grid."""
+    for bh, s in ((1, (1 << 31) - 257), ((1 << 32) - 1, 1), ((1 << 32) - 1, 200), (1 << 31, 70), (7, 1 << 23)):
+        for d in (16, 64):
+            try:
+                sel = route(bh, s, d, False, q=BASE + 2)[1]
+            except nc.NcError:
+                continue
+            assert sel.grid[0] * sel.threads <= 0xFFFFFFFF
