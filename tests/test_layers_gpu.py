@@ -21,11 +21,12 @@ KERNELS = [("d64_q8s1p2t2", 256, 512), ("d64_q4s1p2t2", 128, 256), ("d64_q2s4p2"
 
 @pytest.mark.parametrize("kernel,bm,threads", KERNELS)
 @pytest.mark.parametrize("bh,blocks", [(1, 3), (2, 129), (3, 86), (4, 65), (8, 32), (8, 33), (8, 65), (12, 43), (24, 21),
-                                       (40, 13), (64, 5), (256, 2), (257, 2), (5, 103)])
+                                       (40, 13), (64, 5), (256, 2), (257, 2), (5, 103), (1, 1), (8, 1), (257, 1),
+                                       (1000, 1), (1027, 1), (8, 2), (300, 2), (94, 7)])
 def test_every_block_once(gpu, kernel, bm, threads, bh, blocks):
     """V constant 1 per (head, column) pattern makes O = V whatever the scores, so each row shows whether
     it was written, from its own head; a sentinel shows rows that were not. Grids of just under, at and
-    just over one and two layers of 256 workgroups."""
+    just over one and two layers of 256 workgroups, and one or two blocks per head."""
     d, s = int(kernel[1:3]), blocks * bm - 7
     un = kernel.endswith("_u")
     wl = Workload(f"layers_{kernel}", bh, s, d, True, 1.0 / math.sqrt(d), (("uniform", -1.0, 1.0),) * 3, seed=81)
