@@ -1077,13 +1077,15 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // execute while an MFMA of the same SIMD is in flight (~10 cycles each). The zeros are no barrier
     // to a weight that overflowed or is NaN, so such a tile's sums are not used: its redo adds each
     // lane's own weights by v_dot2c. The private-staging kernels of d = 32 and 64, whose few waves wait
-    // on the tile's serial chain (S^T, weights, sum, PV), lose by the longer one (c3 5.59 -> 5.87 us), and
-    // the `_unaligned` kernels have no check that would keep a NaN in its row: v_dot2c there.
+    // on the tile's serial chain (S^T, weights, sum, PV), lose by the longer one (c3 5.59 -> 5.87 us), and so
+    // do d = 16's on short sequences, with one ring stage (BH=27 S=405 bf16 4.32 -> 4.57 us; with two stages
+    // they gain: BH=3 S=2677 causal 7.12 -> 6.46). The `_unaligned` kernels have no check that would keep
+    // a NaN in its row. v_dot2c in all of these.
     // Measured against v_dot2c (with the first tile's max and one check per tile below): BH=32 S=4096
     // d=64 146.9 -> 139.8 us, BH=64 S=4096 d=64 causal 156.6 -> 146.2, BH=128 S=512 d=64 causal 11.85 ->
     // 10.97, BH=4 S=8192 d=64 causal 54.9 -> 50.9, BH=32 S=4096 d=32 104.8 -> 101.8, BH=64 S=2048 d=16
     // 48.8 -> 45.7.
-    constexpr bool MSUM = !UN && (D == 16 || !PRIV);
+    constexpr bool MSUM = !UN && (!PRIV || (D == 16 && NSTAGE > 1));
     // UN moves the running max to a tile's max ahead of its weights, as the generic kernels that these
     // layouts have otherwise do, and is dispatched with their number of key splits: a row's weights are
     // then rounded at the same maxima, so that the two differ by the rounding of their f32 sums alone.
