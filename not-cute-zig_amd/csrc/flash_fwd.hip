@@ -1086,6 +1086,7 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // 10.97, BH=4 S=8192 d=64 causal 54.9 -> 50.9, BH=32 S=4096 d=32 104.8 -> 101.8, BH=64 S=2048 d=16
     // 48.8 -> 45.7.
     constexpr bool MSUM = !UN && (!PRIV || (D == 16 && NSTAGE > 1));
+    constexpr bool SUM2 = D == 32 && NQ == 4 && !CAUSAL;
     // UN moves the running max to a tile's max ahead of its weights, as the generic kernels that these
     // layouts have otherwise do, and is dispatched with their number of key splits: a row's weights are
     // then rounded at the same maxima, so that the two differ by the rounding of their f32 sums alone.
@@ -1197,10 +1198,13 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
                 }
             }
             if constexpr (MF) {
-                floatx4 z = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks) z = mfma16<BF>(__builtin_bit_cast(half8, ones), pf[ks], z);
-                ls = z[0];
+                // SUM2: two independent products. Chained on each other they made the d=32 q4s1 kernel, with
+                // two workgroups on a CU, 4-5 % slower than v_dot2c was: BH=7 S=7424 101 -> 106 us, BH=20
+                // S=3200 46.4 -> 48.9, independent 46.9. The others are as fast or faster chained (causal 0.4 %).
+                const floatx4 z = {0.f, 0.f, 0.f, 0.f};
+                const floatx4 z0 = mfma16<BF>(__builtin_bit_cast(half8, ones), pf[0], z);
+                const floatx4 z1 = mfma16<BF>(__builtin_bit_cast(half8, ones), pf[1], SUM2 ? z : z0);
+                ls = SUM2 ? z0[0] + z1[0] : z1[0];
             }
             return ls;
         };
