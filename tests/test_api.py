@@ -206,7 +206,7 @@ def test_dispatch_headline_and_large_configs():
 
 
 def test_dispatch_alignment_fallbacks():
-    # odd slice pad (the reference's smoke strides): element-wise kernel
+    # odd slice pad (the reference's smoke strides): `_unaligned` kernel
     sel = nc.select_kernel(nc.options(batch_heads=2, seq_len=32, head_dim=32, q_stride=32 * 32 + 17,
                                       k_stride=32 * 32 + 19, v_stride=32 * 32 + 23, o_stride=32 * 32 + 29,
                                       causal=True))

@@ -114,7 +114,7 @@ def test_element_type_validation_and_dispatch():
         s16, sbf = nc.select_kernel(o16), nc.select_kernel(obf)
         assert sbf.name.decode() == s16.name.decode() + "_bf16"
         assert (tuple(sbf.grid), sbf.threads, sbf.lds_bytes) == (tuple(s16.grid), s16.threads, s16.lds_bytes)
-    # misaligned bases pick the element-wise bf16 twin
+    # misaligned bases pick an `_unaligned` bf16 kernel
     o = Workload(**{**CONFIGS["c3"].__dict__, "dtype": "bf16"}).options()
     sel = nc.select_kernel_for(o, 0x1002, 0x2000, 0x3000, 0x4000)
     assert sel.name.decode().endswith("_unaligned_bf16")

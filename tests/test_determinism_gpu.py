@@ -25,7 +25,8 @@ CASES = [
     (128, 512, 64, True, "f16", 0),   # 4 query waves
     (4, 1500, 32, True, "f16", 0),
     (4, 700, 16, False, "f16", 0),
-    (2, 333, 64, True, "f16", 1),     # element-wise (unaligned) kernels
+    (2, 333, 64, True, "f16", 1),     # an `_unaligned` kernel, private staging
+    (16, 1500, 64, False, "f16", 1),  # one with shared staging
     (8, 1024, 64, True, "bf16", 0),
     (16, 1024, 64, False, "bf16", 0),
 ]
@@ -36,7 +37,7 @@ def test_repeated_runs_are_bitwise_identical(gpu, case):
     bh, s, d, causal, dtype, offset = case
     wl = Workload(f"det_{bh}_{s}_{d}", bh, s, d, causal, 1.0 / math.sqrt(d), (("normal", 0.0, 1.0),) * 3,
                   seed=77 + s, dtype=dtype)
-    sel = nc.select_kernel(wl.options())  # for aligned bases; offset 1 takes the element-wise twin
+    sel = nc.select_kernel(wl.options())  # for aligned bases; offset 1 takes an `_unaligned` kernel
     print(f"[case] {wl.describe()} dtype={dtype} offset={offset} aligned-base kernel={sel.name.decode()}",
           flush=True)
     q, k, v = wl.make_inputs()

@@ -1,7 +1,7 @@
 """GPU parity: the gfx950 kernels through the C ABI (nc_flash_launch) against the CPU oracle.
 
 Cases: the five benchmark configurations (c4/c5 on a deterministic row subset, exact per row), the
-reference's own smoke cases (odd slice pads -> element-wise kernels) and compare cases, ragged
+reference's own smoke cases (odd slice pads -> `_unaligned` kernels) and compare cases, ragged
 sequence lengths around every tile edge, a misaligned base pointer, large logits, determinism and
 padding that must stay untouched.
 """
@@ -88,7 +88,7 @@ def test_ragged_lengths(gpu, d, causal):
 
 @pytest.mark.parametrize("d", [16, 32, 64])
 def test_misaligned_base(gpu, d):
-    """Base pointers one element off 16-byte alignment select the element-wise kernels."""
+    """Base pointers one element off 16-byte alignment select the `_unaligned` kernels."""
     wl = Workload(f"misaligned_d{d}", 2, 77, d, True, 1.0 / math.sqrt(d), (("normal", 0.0, 1.0),) * 3, seed=7)
     _check(gpu, wl, offset=1)
 
