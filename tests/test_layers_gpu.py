@@ -2,7 +2,6 @@
 query block of every head is computed exactly once, whatever the head count, at the edges of the layers."""
 
 import math
-import re
 
 import numpy as np
 import pytest
@@ -13,7 +12,7 @@ from flash_workloads import Workload
 
 pytestmark = pytest.mark.gpu
 
-# (kernel, rows per workgroup, threads, workgroups per CU)
+# (kernel, rows per workgroup, threads)
 KERNELS = [("d64_q8s1p2t2", 256, 512), ("d64_q4s1p2t2", 128, 256), ("d64_q2s4p2", 64, 512), ("d64_q1s8p1", 32, 512),
            ("d32_q4s1p3", 128, 256), ("d16_q4s1p2t2", 128, 256), ("d32_q1s8p2", 32, 512),
            ("d64_q2s2p2_u", 64, 256)]
