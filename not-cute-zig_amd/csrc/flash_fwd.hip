@@ -643,12 +643,14 @@ struct PipeSlot {
     uint32_t L, head, qb_rev;
 };
 
-// Workgroups of a causal pipelined kernel that share a CU from the start of a launch (by its LDS and
-// registers).
-template <int D, int NQ, int NS, int NSTAGE, int SUB>
+// Workgroups of a causal shared-staging kernel that share a CU from the start of a launch, by its LDS and
+// its waves per SIMD (512 VGPRs over what the compiler gives it: d=64 116-123, d=32 82-84, UN 76, d=16
+// 76-80, UN 70; tests/test_layers_gpu.py holds the result against the occupancy of the built kernels).
+template <int D, int NQ, int NS, int NSTAGE, int SUB, bool UN>
 constexpr int pipe_layers() {
     using C = PipeCfg<D, NQ, NS, NSTAGE, SUB>;
-    constexpr int by_lds = 160 * 1024 / C::LDS_BYTES, by_regs = (D == 64 ? 4 : D == 32 || NQ == 1 ? 5 : 6) * 4 / C::NW;
+    constexpr int by_lds = 160 * 1024 / C::LDS_BYTES;
+    constexpr int by_regs = (D == 64 ? 4 : (D == 32 ? 5 : 6) + (UN ? 1 : 0)) * 4 / C::NW;
     return by_lds < by_regs ? by_lds : by_regs;
 }
 
@@ -1671,7 +1673,7 @@ __device__ __forceinline__ void flash_fwd_pipe_kernel(const nc_flash_kernel_args
     flash_fwd_pipe_body<D, NQ, NS, CAUSAL, NSTAGE, SUB, BF, XS, UN>(a, smem, [&](uint32_t bh) {
         // Private staging keeps falling order: its grids are of few layers, and the layers' divisions stand
         // before the first load (12 launches of BH=8 S=128 d=32 43.3 -> 43.1 us, of S=250, odd, 50.9 -> 50.3).
-        constexpr int LAYERS = CAUSAL && NQ > 1 ? pipe_layers<D, NQ, NS, NSTAGE, SUB>() : 1;
+        constexpr int LAYERS = CAUSAL && NQ > 1 ? pipe_layers<D, NQ, NS, NSTAGE, SUB, UN>() : 1;
         return pipe_slot<LAYERS>(blockIdx.x, bh, a.num_q_blocks);
     });
 }

@@ -55,3 +55,16 @@ def test_every_block_once(gpu, kernel, bm, threads, bh, blocks):
     # O = sum(w v) / sum(w) with v constant and the same rounded w in both sums: f32 rounding only
     want = (np.arange(bh) % 61 + 1).astype(np.float32)[:, None, None]
     assert np.max(np.abs(out / want - 1.0)) <= 1e-4
+
+
+# Workgroups per CU that the launch order of each causal shared-staging kernel assumes (pipe_layers)
+LAYERS = {"d64_q8s1p2t2": 2, "d64_q4s1p2t2": 4, "d64_q2s4p2": 2, "d64_q2s2p2_u": 3, "d32_q4s1p3": 5, "d32_q2s4p2": 2,
+          "d32_q2s2p2_u": 6, "d16_q4s1p2t2": 6, "d16_q2s4p2": 3, "d16_q2s2p2_u": 7}
+
+
+@pytest.mark.parametrize("dtype", ["", "_bf16"])
+@pytest.mark.parametrize("kernel", sorted(LAYERS))
+def test_layers_are_the_occupancy(gpu, kernel, dtype):
+    q, s = (int(kernel[kernel.index(c) + 1]) for c in "qs")
+    name = f"nc_flash_fwd_{kernel.replace('_u', '')}_causal" + ("_unaligned" if "_u" in kernel else "") + dtype
+    assert gpu.get_function(name).max_active_blocks(64 * q * s) == LAYERS[kernel]
