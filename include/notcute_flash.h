@@ -259,8 +259,8 @@ typedef struct nc_flash_kernel_selection {
  * at that size, where no packed-slice 3-D grid applies). */
 int nc_flash_select_kernel(const nc_flash_options *opts, nc_flash_kernel_selection *out);
 
-/* Same, for the actual buffers: picks an `_unaligned` variant when a pointer or stride breaks
- * 16-byte alignment (the reference's smoke cases use odd slice pads, src/main.zig:190-193). */
+/* Same, for the actual buffers: picks an `_unaligned` variant, pipelined or generic, when a pointer or
+ * stride breaks 16-byte alignment (the reference's smoke cases use odd slice pads, src/main.zig:190-193). */
 int nc_flash_select_kernel_for(const nc_flash_options *opts, const void *q, const void *k,
                                const void *v, const void *o, nc_flash_kernel_selection *out);
 
@@ -318,7 +318,10 @@ int nc_flash_kernel_scratch_bytes(const char *name, const nc_flash_options *opts
  * stride seq_len*head_dim, every row stride head_dim; selected by nc_flash_select_kernel for such
  * layouts) declare one parameter per field of the block, in order, so that their first seven are
  * preloaded into SGPRs: params[i] = the address of field i, *count = NC_FLASH_MAX_KERNEL_PARAMS. Either
- * way the kernarg segment is the block's bytes. `params` must hold `capacity` >= *count entries and
+ * way the kernarg segment is the block's bytes. The pipelined `_unaligned` kernels (q2s2p2, q1s8p1 and
+ * q1s8p2) take K and V with one and the same even row stride, Q, K and V at any element and O at any
+ * float; launched by name with other K/V row strides they write nothing (the selection takes the generic
+ * `_m64_..._unaligned` kernels there). `params` must hold `capacity` >= *count entries and
  * stays valid while `args` does. NC_ERROR_NOT_FOUND for a name that is not a flash kernel. */
 #define NC_FLASH_MAX_KERNEL_PARAMS 20u
 int nc_flash_kernel_params(const char *name, nc_flash_kernel_args *args, void **params, uint32_t capacity,

@@ -230,9 +230,10 @@ const char *reference_kernel(const nc_flash_options &o) {
 }
 
 // MI355X dispatch (256 CUs): at d = 64 and 32 every pipelined kernel of the head size is priced by a
-// cost model and the cheapest is launched (d = 16: fitted thresholds, in choose_pipe). A kernel's
-// workgroups are dealt to the CUs in block order (heaviest causal query blocks first), so the
-// busiest CU holds workgroups 0, 256, 512, ... . It runs up to
+// cost model and the cheapest is launched (d = 16: fitted thresholds, in choose_pipe). The model deals
+// a kernel's workgroups to the CUs in block order, heaviest causal query blocks first, so that its
+// busiest CU holds workgroups 0, 256, 512, ... . (The causal shared-staging kernels turn every other
+// resident layer since, so their busiest CU holds less; the constants are older too, see below.) It runs up to
 // wg_per_cu of them at once (from each kernel's registers and LDS); each resident workgroup needs
 // rho + steps units of work, steps being its busiest wave's sequential 32-key tiles (the padded key
 // blocks up to its last visible key), and advances one unit per max(lat, k * waves_per_simd * tau)
@@ -241,11 +242,12 @@ const char *reference_kernel(const nc_flash_options &o) {
 // blocks, causal imbalance and how full the CUs are all enter through the steps and the sharing,
 // which fixed grid-size thresholds miss off a power-of-two grid. (a, rho, lat, tau) were fitted per
 // kernel to interleaved GPU timings of every variant on 245 (d=64) and 244 (d=32) shapes (BH 1-1024,
-// S 64-16384, causal and not; a grid, an off-grid set and a random set). On 100 random shapes per
-// head size timed after the fit the picks average 1.003x (d=64) and 1.006x (d=32) the per-shape
-// best, where the threshold rules they replace averaged 1.052x and 1.023x; on 50 bf16 shapes each,
-// 1.010x and 1.006x (thresholds: 1.046x and 1.049x). The bf16 twins have the same instruction
-// stream and use the same model.
+// S 64-16384, causal and not; a grid, an off-grid set and a random set), before the row sum on the matrix
+// cores and the turned layers. With the kernels as they are, on 220 random packed shapes per head size
+// (BH 1-1024, S 64-16384, a quarter bf16) the picks average 1.010x (d=64, worst 1.30x: BH=33 S=2485
+// causal, q2s4 57.8 us for q4s1's 44.5), 1.008x (d=32, 1.17x: BH=28 S=1560, q4s1 25.7 for q2s4's 21.9) and,
+// by the thresholds, 1.011x (d=16) the per-shape best. The bf16 twins have the same instruction stream and
+// use the same model.
 // `balance`: the non-causal kernel orders its waves by remaining work in the grid's last
 // wg_per_cu * CUs workgroups (nc_flash_kernel_args.balance_tail), where that was measured faster.
 struct PipeModel {
@@ -372,9 +374,10 @@ const Variant *choose_pipe_layout(const nc_flash_options &o) {
     const bool causal = o.causal != 0;
     const bool bf = o.element_type == NC_ELEMENT_BF16;
     if (d == 16) {
-        // d = 16 tiles are cheap next to their softmax and staging, and the model above picks worse
+        // d = 16 tiles are cheap next to their softmax and staging, and the model above picked worse
         // there (1.010x the per-shape best in cross-validation) than these fitted thresholds
-        // (1.008-1.011x on two random sets timed after their fit, f16 and bf16): q4s1 from 384-1536 of
+        // (1.008-1.011x on two random sets timed after their fit, f16 and bf16; 1.011x, worst 1.32x at
+        // BH=90 S=152, with the kernels as they are): q4s1 from 384-1536 of
         // its workgroups, more for longer sequences, then q2s4 from 192-768 of its own.
         const uint64_t S = o.seq_len, bh = o.batch_heads;
         const uint64_t w128 = (S + 127) / 128 * bh, w64 = (S + 63) / 64 * bh;

@@ -27,9 +27,9 @@
 //     the workgroup's last query are never staged. Heavy (late) query blocks are dispatched first and
 //     workgroups of the same heads are kept on one XCD so their K/V stay in that XCD's L2.
 //   * exp is v_exp_f32 on log2-scaled scores (scale * log2(e) folded into one multiply).
-// The generic family (flash_fwd_body: 64-bit addressing, and element-wise variants for odd or unequal
-// K/V row strides and unaligned slices of that size) stages K/V through registers and stores V^T transposed in LDS with
-// keys permuted so each A-operand fetch is one ds_read_b128. The pipelined family
+// The generic family (flash_fwd_body: 64-bit addressing, and element-wise variants for odd or unequal K/V
+// row strides, and for other slices off 16-byte alignment where they are faster) stages K/V through
+// registers and stores V^T transposed in LDS with keys permuted so each A-operand fetch is one ds_read_b128. The pipelined family
 // (flash_fwd_pipe_body, the fast path) streams K/V with buffer->LDS DMA into a ring and reads V^T
 // with ds_read_b64_tr_b16; it is described where it is defined.
 //   * Every kernel also exists with a `_bf16` suffix: bf16 Q/K/V, probabilities rounded to bf16 for
@@ -467,7 +467,8 @@ __device__ __forceinline__ void flash_fwd_body(const nc_flash_kernel_args &a) {
 // and PV before the next. Kernels with key-split waves (NS > 1) stage the workgroup's Q rows in LDS
 // once instead of every wave loading its group's rows.
 // The softmax keeps a lazy running max: weights are formed against the max as it stands and the
-// max only moves when a weight overflows (or, before the first tile, when a row has none).
+// max only moves when a weight overflows (or, before the first tile, when a row has none). The UN form
+// takes the max ahead of every tile's weights instead.
 // ---------------------------------------------------------------------------------------------
 
 #define NC_LDS(T) __attribute__((address_space(3))) T
@@ -537,8 +538,8 @@ struct IC {
     static constexpr int value = N;
 };
 
-// x from another lane of the same 16-lane row, selected by the DPP control CTRL (quad_perm,
-// row_half_mirror, row_newbcast); every lane of the wave must be active.
+// x from another lane of the same 16-lane row, selected by the DPP control CTRL (quad_perm, row_shl,
+// row_shr, row_ror, row_half_mirror, row_newbcast); the lanes that x is taken from must be active.
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float x) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, false));
@@ -757,8 +758,8 @@ constexpr int pipe_lds_bytes() {
 // Odd slice pads, us: element-wise generic kernels / staging through registers with a funnel shift
 // per chunk (148-176 VGPRs, half the workgroups per CU) / shifting each chunk in place in LDS / this:
 // BH=8 S=1024 d=64 causal 19.3 / 8.7 / 11.1 / 7.5, BH=32 S=4096 d=64 267 / 209 / 181 / 152, BH=16 S=1500
-// d=64 35.4 / 31.0 / 27.9 / 20.3 (16-byte aligned slices: 5.6, 154, 18.0), all four with a lazy running
-// max; with the exact one (below) the kernels that are kept take 7.5, 207 and 23.2.
+// d=64 35.4 / 31.0 / 27.9 / 20.3 (16-byte aligned slices, v_dot2c row sum: 5.6, 154, 18.0), all four
+// with a lazy running max; with the exact one (below) the kernels that are kept take 7.5, 207 and 23.2.
 template <int D, int NQ, int NS, bool CAUSAL, int NSTAGE, int SUB, bool BF, bool XS = false, bool UN = false,
           typename SlotFn>
 __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &a, char *smem, SlotFn &&slot_of) {
@@ -1086,7 +1087,7 @@ __device__ __forceinline__ void flash_fwd_pipe_body(const nc_flash_kernel_args &
     // Measured against v_dot2c (with the first tile's max and one check per tile below): BH=32 S=4096
     // d=64 146.9 -> 139.8 us, BH=64 S=4096 d=64 causal 156.6 -> 146.2, BH=128 S=512 d=64 causal 11.85 ->
     // 10.97, BH=4 S=8192 d=64 causal 54.9 -> 50.9, BH=32 S=4096 d=32 104.8 -> 101.8, BH=64 S=2048 d=16
-    // 48.8 -> 45.7.
+    // 47.5 -> 45.8.
     constexpr bool MSUM = !UN && (!PRIV || (D == 16 && NSTAGE > 1));
     constexpr bool SUM2 = D == 32 && NQ == 4 && !CAUSAL;
     // UN moves the running max to a tile's max ahead of its weights, as the generic kernels that these
