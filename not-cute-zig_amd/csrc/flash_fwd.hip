@@ -107,10 +107,10 @@ __device__ __forceinline__ float sum2(half2v p, float acc) {
         return __builtin_amdgcn_fdot2(p, ones, acc, false);
     }
 }
-// A 32-key tile's weight sum (per lane, 16 rounded weights) at or above this moves the running max
-// to the tile max. f16: a weight that overflows f16 does, which turns the sum of the rounded
-// weights infinite. bf16 has f32's range, so weights are held below 2^20 to keep the f32 row sum
-// and O accumulators far from overflow.
+// A 32-key tile's weight sum (a lane's 16 rounded weights; on the matrix cores the query's 32) at or above
+// this moves the running max to the tile max. f16: a weight that overflows f16 does, which turns the sum
+// of the rounded weights infinite. bf16 has f32's range, so weights are held below 2^20 to keep the f32
+// row sum and O accumulators far from overflow.
 template <bool BF>
 __device__ __forceinline__ float weight_sum_limit() {
     return BF ? 1048576.0f : __builtin_inff();
