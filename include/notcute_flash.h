@@ -178,7 +178,7 @@ typedef void *nc_graph;
 int nc_stream_begin_capture(nc_stream stream);
 int nc_stream_end_capture(nc_stream stream, nc_graph *out); /* capture + instantiate */
 int nc_graph_launch(nc_graph graph, nc_stream stream);
-int nc_graph_destroy(nc_graph graph);
+int nc_graph_destroy(nc_graph graph); /* no replay of it may be in flight */
 
 /* Name of the plain 16-byte copy kernel in the embedded code object, launched by the benchmark to
  * calibrate rocprofv3 FETCH_SIZE / WRITE_SIZE counters against a known byte count:

@@ -596,10 +596,13 @@ class Event:
 
 
 class Graph:
-    """A captured, instantiated HIP graph (extension; the reference has none)."""
+    """A captured, instantiated HIP graph (extension; the reference has none). A replay is ordered only by
+    the stream it is launched on: a reader of its outputs synchronises that stream or waits for an event
+    recorded there."""
 
     def __init__(self, handle: int):
         self.handle = handle
+        self._streams = set()
 
     @classmethod
     def capture(cls, stream: "Stream", body) -> "Graph":
@@ -614,12 +617,20 @@ class Graph:
         return cls(int(h.value))
 
     def launch(self, stream: "Stream") -> None:
+        self._streams.add(stream)
         check(lib().nc_graph_launch(self.handle, stream.handle), "Graph.launch")
 
     def destroy(self) -> None:
+        """Waits for the replays in flight (on streams that still exist) first: they use the graph and the
+        buffers captured in it, which callers release next."""
         if self.handle:
-            check(lib().nc_graph_destroy(self.handle), "Graph.destroy")
-            self.handle = 0
+            try:
+                for stream in self._streams:
+                    if stream.handle:
+                        stream.synchronize()
+            finally:
+                check(lib().nc_graph_destroy(self.handle), "Graph.destroy")
+                self.handle = 0
 
 
 def flash_launch(module: Module, q: DeviceBuffer, k: DeviceBuffer, v: DeviceBuffer, o: DeviceBuffer,

@@ -584,3 +584,40 @@ def test_kernel_params_forms():
     with pytest.raises(nc.NcError) as e:
         nc.kernel_params("flash_attention_fwd_v2", a)
     assert e.value.name == "NotFound"
+
+
+def test_a_graph_is_destroyed_after_its_replays(monkeypatch):
+    """destroy() waits for every stream the graph was replayed on, but not for one that is gone, and
+    destroys the graph also when waiting fails."""
+    calls, fail = [], set()
+
+    class Calls:
+        def __getattr__(self, name):
+            def call(*args):
+                calls.append((name, args[0]))
+                return 1 if name in fail else 0
+            return call
+
+    monkeypatch.setattr(nc, "lib", lambda: Calls())
+    monkeypatch.setattr(nc, "check", lambda st, what: (_ for _ in ()).throw(RuntimeError(what)) if st else None)
+    streams = []
+    for handle in (11, 12, 13):
+        s = nc.Stream.__new__(nc.Stream)
+        s.handle = handle
+        streams.append(s)
+    graph = nc.Graph(7)
+    for s in streams * 2:
+        graph.launch(s)
+    streams[2].handle = 0
+    calls.clear()
+    graph.destroy()
+    assert sorted(calls[:-1]) == [("nc_stream_synchronize", 11), ("nc_stream_synchronize", 12)]
+    assert calls[-1] == ("nc_graph_destroy", 7) and graph.handle == 0
+    graph.destroy()  # once
+    assert len(calls) == 3
+    graph = nc.Graph(8)
+    graph.launch(streams[0])
+    fail.add("nc_stream_synchronize")
+    with pytest.raises(RuntimeError):
+        graph.destroy()
+    assert calls[-1] == ("nc_graph_destroy", 8) and graph.handle == 0
